@@ -116,6 +116,168 @@ __global__ void store_weight_kernel(const float* w, int64_t rows, int64_t cols, 
   }
 }
 
+// Permuted rows: the row is read in order into LDS and gathered from there.
+// A gather straight from global memory touches a 64-byte line per element and
+// lane; from LDS the memory traffic is the rows themselves.  A workgroup
+// takes `nr` rows so that the permutation is read once for all of them (nr
+// rows of LDS words, at most PERM_LDS bytes, two workgroups per CU).
+// Bound by HBM; measured, 14336 x 4096 with codes: load 191 -> 74 us (4.8
+// TB/s), store 457 -> 95 us (5.0 TB/s).
+constexpr int PERM_NT = 512;
+constexpr int64_t PERM_LDS = 64 << 10;  // LDS bytes of the staged rows
+
+// Rows per workgroup for rows of `bytes` LDS bytes; 0: too wide to stage.
+inline int perm_rows(int64_t bytes) {
+  const int64_t n = PERM_LDS / bytes;
+  return (int)(n > 8 ? 8 : n);
+}
+
+// out[r][j] = dead[j] ? 0 : w[r][perm[j]], rows nr blockIdx.x .. (matrix
+// blockIdx.z as load_weight_kernel)
+template <typename T>
+__global__ __launch_bounds__(PERM_NT) void load_weight_perm_kernel(const T* w, int64_t rows, int64_t cols, int64_t ldw,
+                                                                   const int32_t* perm, const int32_t* dead,
+                                                                   float* out, int64_t sw, int64_t sp, int nr) {
+  extern __shared__ __attribute__((aligned(16))) char perm_smem[];
+  T* lw = reinterpret_cast<T*>(perm_smem);
+  const int64_t z = blockIdx.z;
+  w += z * sw;
+  perm += z * sp;
+  if (dead) dead += z * cols;
+  out += z * rows * cols;
+  const int64_t r0 = (int64_t)blockIdx.x * nr;
+  const int n = (int)(rows - r0 < nr ? rows - r0 : nr);
+  constexpr int V = 16 / sizeof(T);
+  if (cols % V == 0 && ldw % V == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0) {
+    for (int r = 0; r < n; ++r)
+      for (int64_t j = (int64_t)threadIdx.x * V; j < cols; j += PERM_NT * V)
+        *reinterpret_cast<u32x4_t*>(lw + r * cols + j) = *reinterpret_cast<const u32x4_t*>(w + (r0 + r) * ldw + j);
+  } else {
+    for (int r = 0; r < n; ++r)
+      for (int64_t j = threadIdx.x; j < cols; j += PERM_NT) lw[r * cols + j] = w[(r0 + r) * ldw + j];
+  }
+  __syncthreads();
+  const bool vec = (cols & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+  for (int64_t j4 = (int64_t)threadIdx.x * 4; j4 < cols; j4 += PERM_NT * 4) {
+    int src[4];
+    bool off[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int64_t j = j4 + e < cols ? j4 + e : cols - 1;
+      src[e] = perm[j];
+      off[e] = dead && dead[j];
+    }
+    for (int r = 0; r < n; ++r) {
+      f32x4_t v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const T x = lw[r * cols + src[e]];
+        v[e] = off[e] ? 0.f : sizeof(T) == 2 ? bf16_bits_to_f32((uint16_t)x) : __uint_as_float((uint32_t)x);
+      }
+      float* o = out + (r0 + r) * cols + j4;
+      if (vec) {
+        *reinterpret_cast<f32x4_t*>(o) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (j4 + e < cols) o[e] = v[e];
+      }
+    }
+  }
+}
+
+// out[r][j] = w[r][invperm[j]] (and the codes likewise) for rows nr
+// blockIdx.x ..; a staged word holds the bf16 bits and the code above them,
+// or, for fp32 (BF16 false), the value with the codes' bytes behind the rows.
+template <bool BF16>
+__global__ __launch_bounds__(PERM_NT) void store_weight_perm_kernel(const float* w, int64_t rows, int64_t cols,
+                                                                    const int32_t* invperm, void* out,
+                                                                    int64_t ld_out, const int8_t* cin, int8_t* cout,
+                                                                    int64_t sp, int64_t so, int nr) {
+  extern __shared__ __attribute__((aligned(16))) char perm_smem[];
+  uint32_t* lw = reinterpret_cast<uint32_t*>(perm_smem);
+  int8_t* lc = reinterpret_cast<int8_t*>(lw + (int64_t)nr * cols);
+  const int64_t z = blockIdx.z;
+  w += z * rows * cols;
+  invperm += z * sp;
+  uint16_t* ob = static_cast<uint16_t*>(out) + z * so;
+  float* of = static_cast<float*>(out) + z * so;
+  const bool codes = cin && cout;
+  if (codes) {
+    cin += z * rows * cols;
+    cout += z * rows * cols;
+  }
+  const int64_t r0 = (int64_t)blockIdx.x * nr;
+  const int n = (int)(rows - r0 < nr ? rows - r0 : nr);
+  // the rows are consecutive: one run of n cols elements
+  const float* wr = w + r0 * cols;
+  const int8_t* cr = cin + r0 * cols;
+  const int64_t total = (int64_t)n * cols;
+  const bool vin = (cols & 3) == 0 && (reinterpret_cast<uintptr_t>(wr) & 15) == 0 &&
+                   (!codes || (reinterpret_cast<uintptr_t>(cr) & 3) == 0);
+  auto stage = [&](int64_t i, float x, uint32_t c) __attribute__((always_inline)) {
+    if (BF16) {
+      lw[i] = f32_to_bf16_bits(x) | (c << 16);
+    } else {
+      lw[i] = __float_as_uint(x);
+      if (codes) lc[i] = (int8_t)c;
+    }
+  };
+  if (vin) {
+    for (int64_t i = (int64_t)threadIdx.x * 4; i < total; i += PERM_NT * 4) {
+      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(wr + i);
+      const uint32_t c = codes ? *reinterpret_cast<const uint32_t*>(cr + i) : 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) stage(i + e, x[e], (c >> (8 * e)) & 0xffu);
+    }
+  } else {
+    for (int64_t i = threadIdx.x; i < total; i += PERM_NT) stage(i, wr[i], codes ? (uint8_t)cr[i] : 0u);
+  }
+  __syncthreads();
+  const bool vout = (cols & 3) == 0 && (ld_out & 3) == 0 && (reinterpret_cast<uintptr_t>(ob) & 7) == 0 &&
+                    (BF16 || (reinterpret_cast<uintptr_t>(of) & 15) == 0) &&
+                    (!codes || (reinterpret_cast<uintptr_t>(cout) & 3) == 0);
+  for (int64_t j4 = (int64_t)threadIdx.x * 4; j4 < cols; j4 += PERM_NT * 4) {
+    int src[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) src[e] = invperm[j4 + e < cols ? j4 + e : cols - 1];
+    for (int r = 0; r < n; ++r) {
+      uint32_t v[4], c[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t i = (int64_t)r * cols + src[e];
+        v[e] = lw[i];
+        c[e] = BF16 ? v[e] >> 16 : codes ? (uint8_t)lc[i] : 0u;
+      }
+      const int64_t ro = (r0 + r) * ld_out + j4, rc = (r0 + r) * cols + j4;
+      if (vout) {
+        if (BF16) {
+          uint2 u;
+          u.x = (v[0] & 0xffffu) | (v[1] << 16);
+          u.y = (v[2] & 0xffffu) | (v[3] << 16);
+          *reinterpret_cast<uint2*>(ob + ro) = u;
+        } else {
+          const u32x4_t u = {v[0], v[1], v[2], v[3]};
+          *reinterpret_cast<u32x4_t*>(of + ro) = u;
+        }
+        if (codes)
+          *reinterpret_cast<uint32_t*>(cout + rc) =
+              (c[0] & 0xffu) | (c[1] & 0xffu) << 8 | (c[2] & 0xffu) << 16 | c[3] << 24;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (j4 + e < cols) {
+            if (BF16)
+              ob[ro + e] = (uint16_t)v[e];
+            else
+              of[ro + e] = __uint_as_float(v[e]);
+            if (codes) cout[rc + e] = (int8_t)c[e];
+          }
+      }
+    }
+  }
+}
+
 inline dim3 grid_rows(int64_t rows, int64_t cols, int64_t batch = 1) {
   int64_t gx = (cols / 4 + 255) / 256;
   if (gx < 1) gx = 1;
@@ -142,9 +304,23 @@ extern "C" int mi355q_gptq_load_weight_batched(const void* w_dev, mi355q_dtype w
   MQ_CHECK_ARG(w_dtype == MI355Q_BF16 || w_dtype == MI355Q_F32, "gptq_load_weight: dtype must be bf16 or fp32");
   MQ_CHECK_ARG(rows <= 65535 && batch <= 65535, "gptq_load_weight: at most 65535 rows and matrices");
   MQ_CHECK_ARG(batch == 1 || stride_w >= rows * ldw, "gptq_load_weight: matrices overlap");
-  hipLaunchKernelGGL(load_weight_kernel, grid_rows(rows, cols, batch), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), w_dev, w_dtype, rows, cols, ldw, perm_dev, dead_dev,
-                     w_work_dev, stride_w, stride_perm);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  // a permutation gathers from rows staged in LDS, unless a row is too wide
+  // for that (then straight from memory: 2.6 and 4.8 times the time)
+  const int64_t row_bytes = cols * (w_dtype == MI355Q_BF16 ? 2 : 4);
+  const int nr = perm_dev ? perm_rows(row_bytes) : 0;
+  const dim3 pgrid((unsigned)(nr ? (rows + nr - 1) / nr : 1), 1, (unsigned)batch);
+  if (nr && w_dtype == MI355Q_BF16)
+    hipLaunchKernelGGL(load_weight_perm_kernel<uint16_t>, pgrid, dim3(PERM_NT), (size_t)(nr * row_bytes), st,
+                       static_cast<const uint16_t*>(w_dev), rows, cols, ldw, perm_dev, dead_dev, w_work_dev, stride_w,
+                       stride_perm, nr);
+  else if (nr)
+    hipLaunchKernelGGL(load_weight_perm_kernel<uint32_t>, pgrid, dim3(PERM_NT), (size_t)(nr * row_bytes), st,
+                       static_cast<const uint32_t*>(w_dev), rows, cols, ldw, perm_dev, dead_dev, w_work_dev, stride_w,
+                       stride_perm, nr);
+  else
+    hipLaunchKernelGGL(load_weight_kernel, grid_rows(rows, cols, batch), dim3(256), 0, st, w_dev, w_dtype, rows, cols,
+                       ldw, perm_dev, dead_dev, w_work_dev, stride_w, stride_perm);
   MQ_LAUNCH_CHECK();
   return MI355Q_OK;
 }
@@ -271,9 +447,23 @@ extern "C" int mi355q_gptq_store_weight_batched(const float* w_work_dev, int64_t
   MQ_CHECK_ARG(codes_out_dev != codes_in_dev || !codes_in_dev, "gptq_store_weight: codes must not alias");
   MQ_CHECK_ARG(rows <= 65535 && batch <= 65535, "gptq_store_weight: at most 65535 rows and matrices");
   MQ_CHECK_ARG(batch == 1 || stride_out >= rows * ld_out, "gptq_store_weight: matrices overlap");
-  hipLaunchKernelGGL(store_weight_kernel, grid_rows(rows, cols, batch), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), w_work_dev, rows, cols, invperm_dev, w_out_dev,
-                     out_dtype, ld_out, codes_in_dev, codes_out_dev, stride_perm, stride_out);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const bool bf16 = out_dtype == MI355Q_BF16;
+  const int64_t row_bytes = cols * (bf16 ? 4 : 5);
+  const int nr = invperm_dev ? perm_rows(row_bytes) : 0;
+  const dim3 pgrid((unsigned)(nr ? (rows + nr - 1) / nr : 1), 1, (unsigned)batch);
+  if (nr && bf16)
+    hipLaunchKernelGGL(store_weight_perm_kernel<true>, pgrid, dim3(PERM_NT), (size_t)(nr * row_bytes), st, w_work_dev,
+                       rows, cols, invperm_dev, w_out_dev, ld_out, codes_in_dev, codes_out_dev, stride_perm,
+                       stride_out, nr);
+  else if (nr)
+    hipLaunchKernelGGL(store_weight_perm_kernel<false>, pgrid, dim3(PERM_NT), (size_t)(nr * row_bytes), st, w_work_dev,
+                       rows, cols, invperm_dev, w_out_dev, ld_out, codes_in_dev, codes_out_dev, stride_perm,
+                       stride_out, nr);
+  else
+    hipLaunchKernelGGL(store_weight_kernel, grid_rows(rows, cols, batch), dim3(256), 0, st, w_work_dev, rows, cols,
+                       invperm_dev, w_out_dev, out_dtype, ld_out, codes_in_dev, codes_out_dev, stride_perm,
+                       stride_out);
   MQ_LAUNCH_CHECK();
   return MI355Q_OK;
 }
