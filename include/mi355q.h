@@ -96,8 +96,11 @@ int mi355q_hessian_syrk_scaled_bf16(const void* x_dev, int64_t n_tokens, int64_t
 /* The same for calibration activations of any floating type the reference
  * accepts (it casts the input to fp32, modifiers/gptq/gptq_quantize.py:93,
  * modifiers/pruning/sparsegpt/sgpt_sparsify.py:51): bf16 and fp16 take the
- * 16-bit MFMA kernels above (products exact in fp32), fp32 an fp32 MFMA
- * product over the upper tiles (no workspace).  H = beta * H + alpha * X^T X
+ * 16-bit MFMA kernels above (products exact in fp32), fp32 the same kernel on
+ * the rows' three bf16 planes (six products, each sum accurate as in fp32)
+ * from 512 rows and 512 columns on, with the queried workspace; else, without
+ * a workspace, and for values the planes do not hold, an fp32 MFMA product
+ * over the upper tiles.  H = beta * H + alpha * X^T X
  * on the upper triangle, as mi355q_hessian_syrk_scaled_bf16.  x is [n_tokens,
  * d] row-major (ldx); for the 16-bit types d % 8 == 0, ldx % 8 == 0 and x
  * 16-byte aligned.  Workspace: mi355q_hessian_syrk_workspace_size. */
@@ -118,7 +121,7 @@ int mi355q_hessian_syrk(const void* x_dev, mi355q_dtype dtype, int64_t n_tokens,
  * segment starts a new 32-row stage, so segments whose row counts are
  * multiples of 32 give bit for bit the sums of one call over their
  * concatenation.  Workspace: mi355q_hessian_syrk_segments_workspace_size
- * (0 for fp32, which runs one fp32 product per segment). */
+ * (0 for fp32, which runs one fp32 MFMA product per segment). */
 size_t mi355q_hessian_syrk_segments_workspace_size(const int64_t* n_tokens, int n_segments, int64_t d,
                                                    mi355q_dtype dtype);
 int mi355q_hessian_syrk_segments(const void* const* x_devs, const int64_t* n_tokens, int n_segments,

@@ -99,6 +99,9 @@ struct SyrkParams {
   int T;                   // upper tiles per matrix
   float* h0;               // H of expert 0 (leading dimension d)
   int64_t h_stride;
+  // split mode (fp32 rows as three bf16 planes, see SplitPlan)
+  int64_t plane;           // elements between the planes
+  const int* unsafe;       // nonzero: the planes do not hold the rows' values, nothing is done
 };
 
 // Dense syrk over rows held in separate buffers (the calls a Hessian hook
@@ -399,7 +402,16 @@ __device__ __forceinline__ bf16x8_t tr_pair(const char* lds, int off0, int off1)
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-enum StreamMode { kDense = 0, kGrouped = 1, kGroupedGather = 2, kDenseSeg = 3 };
+enum StreamMode { kDense = 0, kGrouped = 1, kGroupedGather = 2, kDenseSeg = 3, kDenseSplit = 4 };
+
+// fp32 rows as products of bf16 planes: v = h + m + l exactly (24 bits of
+// significand in 3 x 8), and v w = h h' + h m' + m h' + h l' + l h' + m m'
+// but for terms below 2^-24 |v w| each.  The six plane products of every
+// kSplitStages stages (128 tokens) follow each other in the stage sequence,
+// so that the planes' rows stay in L2 between them.
+constexpr int kSplitStages = 4, kSplitPairs = 6, kSplitTokens = kSplitStages * 32;
+// (four bits per pair: the planes of the A and of the B operand)
+constexpr uint32_t kSplitA = 0x120100u, kSplitB = 0x102010u;
 
 // One work item of the streaming kernel: tile t of matrix `mat` over token
 // split s (and part `part` of `nparts` for dense tail tiles), into partial
@@ -528,7 +540,17 @@ __device__ __forceinline__ void stream_item(const SyrkParams& p, char* ring, int
   }
   // stage sc of this item: its first token row and how many of its SK rows
   // exist (>= SK: a whole stage)
-  auto stage_rows = [&](int64_t sc, const char*& xs, int64_t& avail) __attribute__((always_inline)) {
+  // (xs: the row's A operand, xt: its B operand, the same row but in split mode)
+  auto stage_rows = [&](int64_t sc, const char*& xs, const char*& xt, int64_t& avail) __attribute__((always_inline)) {
+    if constexpr (MODE == kDenseSplit) {
+      const uint32_t G = (uint32_t)(st_begin + sc), c = G / (kSplitPairs * kSplitStages);
+      const uint32_t r = G - c * (kSplitPairs * kSplitStages), q = r / kSplitStages;
+      const char* x0 = reinterpret_cast<const char*>(p.x) + (int64_t)(c * kSplitStages + r % kSplitStages) * sbytes;
+      xs = x0 + (int64_t)((kSplitA >> (4 * q)) & 15u) * p.plane * 2;
+      xt = x0 + (int64_t)((kSplitB >> (4 * q)) & 15u) * p.plane * 2;
+      avail = SK;   // whole stages: the planes' last rows are zeros
+      return;
+    }
     if constexpr (MODE == kDenseSeg) {
       const int64_t G = st_begin + sc;
       while (G >= seg_e && sk + 1 < sg->n) {
@@ -542,6 +564,7 @@ __device__ __forceinline__ void stream_item(const SyrkParams& p, char* ring, int
       xs = xbase + sc * sbytes;
       avail = n - (st_begin + sc) * SK;
     }
+    xt = xs;
   };
   // Per-lane global addresses of the NDMA DMAs of a stage (A0, B0, A1, B1, ...):
   // lanes past n or d read the zero chunk.
@@ -561,11 +584,11 @@ __device__ __forceinline__ void stream_item(const SyrkParams& p, char* ring, int
         ad[2 * j + 1] = bok ? (const void*)(xr + fb0 * 2) : (const void*)kZeroChunk;
       }
     } else {
-      const char* xs;
+      const char *xs, *xt;
       int64_t avail;
-      stage_rows(sc, xs, avail);
+      stage_rows(sc, xs, xt, avail);
       const char* xa = xs + fa0 * 2;
-      const char* xb = xs + fb0 * 2;
+      const char* xb = xt + fb0 * 2;
       if (fast_ok && avail >= SK) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -586,14 +609,14 @@ __device__ __forceinline__ void stream_item(const SyrkParams& p, char* ring, int
   };
   auto issue = [&](int64_t stage, int slot) __attribute__((always_inline)) {
     const int64_t sc = stage < nst ? stage : nst - 1;
-    const char* xs = nullptr;
+    const char *xs = nullptr, *xt = nullptr;
     int64_t avail = 0;
-    if constexpr (MODE != kGroupedGather) stage_rows(sc, xs, avail);
+    if constexpr (MODE != kGroupedGather) stage_rows(sc, xs, xt, avail);
     if (fast_ok && avail >= SK) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         dma_s(doff[j], xs + fa0 * 2, sa[slot] + 1024u * j);
-        dma_s(doff[j], xs + fb0 * 2, sb[slot] + 1024u * j);
+        dma_s(doff[j], xt + fb0 * 2, sb[slot] + 1024u * j);
       }
     } else {
       const void* ad[NDMA];
@@ -715,7 +738,7 @@ __device__ __forceinline__ void stream_item(const SyrkParams& p, char* ring, int
 
   if (slot < 0) {
     const bool diag = ti == tj;
-    const int64_t ldh = (MODE == kDense || MODE == kDenseSeg) ? p.ldh : p.d;
+    const int64_t ldh = (MODE == kDense || MODE == kDenseSeg || MODE == kDenseSplit) ? p.ldh : p.d;
     if (p.beta == 0.f) {
       // H not read: each accumulator register goes straight to its row of H
       // (a store covers 32 consecutive columns of two rows, lanes 0..31 and
@@ -855,7 +878,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void syrk_stream_kernel(SyrkParams p
   __shared__ __attribute__((aligned(1024))) char ring[8 * SOP];
   // row indices of a gathered chunk
   __shared__ int ridx[MODE == kGroupedGather ? kChunkTokens : 1];
-  if constexpr (MODE == kDense || MODE == kDenseSeg) {
+  if constexpr (MODE == kDense || MODE == kDenseSeg || MODE == kDenseSplit) {
+    if (MODE == kDenseSplit && *p.unsafe != 0) return;
     const int S = p.S;
     int t, s, part = 0, nparts = 1;
     int64_t slot;
@@ -962,7 +986,8 @@ template <int WAVES>
 __global__ __launch_bounds__(NT) void syrk_stream_reduce_kernel(const float* __restrict__ ws, int S,
                                                                 int tail_start, int tail_f, Matrix single,
                                                                 int64_t d, int64_t ldh, int nt, float alpha,
-                                                                float beta) {
+                                                                float beta, const int* unsafe) {
+  if (unsafe && *unsafe != 0) return;
   constexpr int TM = 256, TILE = TM * TM;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t = blockIdx.x;
@@ -1215,6 +1240,18 @@ int choose_splits(int64_t n, int T, int cus) {
   int best = 1;
   for (int k = 2; k <= S; k *= 2)
     if (rounds_x4(k) < rounds_x4(best)) best = k;
+  // A call whose tiles leave CUs idle in one round is split further, down to
+  // 8 stages of 32 tokens a split, while the stages saved (0.7 us each)
+  // outweigh the reduction (about 8 us, and 0.1 us to write and read a
+  // partial tile).  Measured against splits of at least 2048 tokens: 2048 x
+  // 256 51 -> 24 us, 2048 x 512 46 -> 27, 2048 x 1024 47 -> 33, 4096 x 1024
+  // 48 -> 34, 2048 x 2048 49 -> 32, 4096 x 2048 53 -> 40.
+  const int64_t stages = (n + 31) / 32;
+  const auto cost = [T, stages](int k) {
+    return 0.7 * (double)((stages + k - 1) / k) + (k > 1 ? 8.0 + 0.1 * T * k : 0.0);
+  };
+  for (int k = 2 * best; k <= 8 && T * k <= cus && 8 * k <= stages; k *= 2)
+    if (cost(k) < cost(best)) best = k;
   return best;
 }
 
@@ -1292,6 +1329,49 @@ void launch_reduce(const float* ws, int S, const Matrix& single, int64_t d, int6
                        nt, alpha, beta);
 }
 
+// The three bf16 planes of np rows of fp32 x (rows n .. np - 1 and columns d
+// .. ld - 1 zeros), eight columns per thread: h = bf16(v), m = bf16(v - h), l
+// = v - h - m, each difference exact.  Sets *unsafe for a value that this
+// does not represent: not finite, or rounding to infinity in bf16.
+__global__ __launch_bounds__(256) void split_planes_kernel(const float* __restrict__ x, int64_t n, int64_t d,
+                                                           int64_t ldx, uint16_t* __restrict__ out, int64_t np,
+                                                           int64_t ld, int vec, int* unsafe) {
+  const int64_t per = ld / 8;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= np * per) return;
+  const int64_t r = i / per, c = 8 * (i - r * per);
+  float v[8];
+  if (r < n && vec && c + 8 <= d) {
+    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(x + r * ldx + c);
+    const f32x4_t b = *reinterpret_cast<const f32x4_t*>(x + r * ldx + c + 4);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = a[k];
+      v[k + 4] = b[k];
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = r < n && c + k < d ? x[r * ldx + c + k] : 0.f;
+  }
+  u32x4_t o[3];
+  bool bad = false;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint16_t h = f32_to_bf16_bits(v[k]);
+    bad |= (h & 0x7f80u) == 0x7f80u;
+    const float rest = v[k] - bf16_bits_to_f32(h);
+    const uint16_t m = f32_to_bf16_bits(rest);
+    const uint16_t l = f32_to_bf16_bits(rest - bf16_bits_to_f32(m));
+    const uint16_t part[3] = {h, m, l};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) o[q][k / 2] = k & 1 ? o[q][k / 2] | ((uint32_t)part[q] << 16) : part[q];
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4_t*>(out + (q * np + r) * ld + c) = o[q];
+  if (bad) atomicOr(unsafe, 1);
+}
+__global__ void clear_word_kernel(int* p) { *p = 0; }
+
 // H[i][j] *= beta on the upper triangle (a call without tokens)
 __global__ void scale_upper_kernel(float* h, int64_t d, int64_t ldh, float beta) {
   const int64_t i = blockIdx.y;
@@ -1363,7 +1443,8 @@ int hessian16_impl(const void* x_dev, bool f16, int64_t n_tokens, int64_t d, int
   if (S > 1) {
     if (tile_edge(d) == 256)  // the streaming kernel's slots
       hipLaunchKernelGGL(syrk_stream_reduce_kernel<kStreamWaves>, dim3((unsigned)T, 256 / ((NT / 64) * RED_CPW)), dim3(NT), 0,
-                         st, p.ws, S, pl.tail_start, pl.tail_f, p.single, d, ldh, nt, alpha, beta);
+                         st, p.ws, S, pl.tail_start, pl.tail_f, p.single, d, ldh, nt, alpha, beta,
+                         (const int*)nullptr);
     else
       launch_reduce(p.ws, S, p.single, d, ldh, nt, alpha, beta, (unsigned)T, st);
     MQ_LAUNCH_CHECK();
@@ -1473,7 +1554,8 @@ int hessian_seg_impl(const void* const* xs, const int64_t* rows, int nseg, mi355
       MQ_LAUNCH_CHECK();
       if (pl.S > 1) {
         hipLaunchKernelGGL(syrk_stream_reduce_kernel<kStreamWaves>, dim3((unsigned)pl.T, 256 / ((NT / 64) * RED_CPW)),
-                           dim3(NT), 0, st, p.ws, pl.S, pl.tail_start, pl.tail_f, p.single, d, ldh, nt, alpha, b);
+                           dim3(NT), 0, st, p.ws, pl.S, pl.tail_start, pl.tail_f, p.single, d, ldh, nt, alpha, b,
+                           (const int*)nullptr);
         MQ_LAUNCH_CHECK();
       }
     }
@@ -1491,8 +1573,75 @@ extern "C" int mi355q_hessian_syrk_scaled_bf16(const void* x_dev, int64_t n_toke
                         stream);
 }
 
+namespace {
+// fp32 rows on the 16-bit MFMA kernel: six bf16 plane products (see
+// kDenseSplit) in calls of at most `tokens` rows, whose planes take at most
+// about 1 GiB.  Taken from 512 rows and 512 columns on: there the six
+// products, the split (10 us for 1024 x 4096, at HBM speed) and the two
+// launches around them win (fp32 product against planes: 512 x 512 51 / 36
+// us, 512 x 4096 177 / 93, 4096 x 1000 391 / 64, 8192 x 4096 2540 / 836, i.e.
+// 164 TFLOP/s; 256 x 4096 would be a tie).
+// Workspace: a flag, the planes, the partial slots.
+struct SplitPlan {
+  int64_t tokens = 0, np = 0, ld = 0;   // rows per call, padded rows and columns of a plane
+  size_t planes = 0, total = 0;         // byte offset of the slots; all bytes
+};
+constexpr size_t kSplitHead = 256;
+SplitPlan split_plan(int64_t n, int64_t d) {
+  SplitPlan s;
+  if (n < 512 || d < 512) return s;
+  s.ld = (d + 7) / 8 * 8;
+  if (s.ld > (int64_t(1) << 24)) return s;
+  const auto pad = [](int64_t v) { return (v + kSplitTokens - 1) / kSplitTokens * kSplitTokens; };
+  int64_t most = (int64_t(1) << 30) / (6 * s.ld) / kSplitTokens * kSplitTokens;
+  if (most < 4096) most = 4096;
+  s.tokens = n < most ? n : most;
+  s.np = pad(s.tokens);
+  s.planes = kSplitHead + (size_t)3 * s.np * s.ld * 2;
+  s.total = s.planes + mi355q_hessian_workspace_size(kSplitPairs * s.np, d);
+  const int64_t rest = n % s.tokens;   // the last, shorter call may split its tokens another way
+  if (rest) {
+    const size_t t = s.planes + mi355q_hessian_workspace_size(kSplitPairs * pad(rest), d);
+    if (t > s.total) s.total = t;
+  }
+  return s;
+}
+
+int hessian_split_impl(const float* x, int64_t n, int64_t d, int64_t ldx, float* h, int64_t ldh, float alpha,
+                       float beta, const SplitPlan& s, char* ws, hipStream_t st) {
+  int* unsafe = reinterpret_cast<int*>(ws);
+  uint16_t* planes = reinterpret_cast<uint16_t*>(ws + kSplitHead);
+  const int vec = ldx % 4 == 0 && aligned16(x);
+  const int nt = tiles_per_edge(d);
+  for (int64_t r = 0; r < n; r += s.tokens) {
+    const int64_t rows = n - r < s.tokens ? n - r : s.tokens;
+    const int64_t np = (rows + kSplitTokens - 1) / kSplitTokens * kSplitTokens;
+    const float b = r == 0 ? beta : 1.f;
+    hipLaunchKernelGGL(clear_word_kernel, dim3(1), dim3(1), 0, st, unsafe);
+    hipLaunchKernelGGL(split_planes_kernel, dim3((unsigned)((np * (s.ld / 8) + 255) / 256)), dim3(256), 0, st,
+                       x + r * ldx, rows, d, ldx, planes, np, s.ld, vec, unsafe);
+    const int64_t ne = kSplitPairs * np;
+    const DensePlan pl = plan_dense(ne, d);
+    SyrkParams p = dense_params(planes, ne, d, s.ld, h, ldh, alpha, b, pl, ws + s.planes);
+    p.plane = np * s.ld;
+    p.unsafe = unsafe;
+    hipLaunchKernelGGL((syrk_stream_kernel<false, kDenseSplit, kStreamWaves>), dim3((unsigned)pl.grid), dim3(SNT), 0,
+                       st, p, SegArg<kDenseSplit>{});
+    if (pl.S > 1)
+      hipLaunchKernelGGL(syrk_stream_reduce_kernel<kStreamWaves>, dim3((unsigned)pl.T, 256 / ((NT / 64) * RED_CPW)),
+                         dim3(NT), 0, st, p.ws, pl.S, pl.tail_start, pl.tail_f, p.single, d, ldh, nt, alpha, b,
+                         (const int*)unsafe);
+    MQ_LAUNCH_CHECK();
+    // rows with such values: the fp32 product instead
+    const int rc = syrk_f32_upper(x + r * ldx, rows, d, ldx, h, ldh, alpha, b, st, unsafe);
+    if (rc != MI355Q_OK) return rc;
+  }
+  return MI355Q_OK;
+}
+}  // namespace
+
 extern "C" size_t mi355q_hessian_syrk_workspace_size(int64_t n_tokens, int64_t d, mi355q_dtype dtype) {
-  return dtype == MI355Q_F32 ? 0 : mi355q_hessian_workspace_size(n_tokens, d);
+  return dtype == MI355Q_F32 ? split_plan(n_tokens, d).total : mi355q_hessian_workspace_size(n_tokens, d);
 }
 
 extern "C" int mi355q_hessian_syrk(const void* x_dev, mi355q_dtype dtype, int64_t n_tokens, int64_t d, int64_t ldx,
@@ -1514,6 +1663,10 @@ extern "C" int mi355q_hessian_syrk(const void* x_dev, mi355q_dtype dtype, int64_
     return MI355Q_OK;
   }
   MQ_CHECK_ARG(x_dev != nullptr, "hessian: null x");
+  const SplitPlan sp = split_plan(n_tokens, d);
+  if (sp.total > 0 && workspace_dev != nullptr && aligned16(workspace_dev) && workspace_bytes >= sp.total)
+    return hessian_split_impl(static_cast<const float*>(x_dev), n_tokens, d, ldx, h_dev, ldh, alpha, beta, sp,
+                              static_cast<char*>(workspace_dev), st);
   return syrk_f32_upper(static_cast<const float*>(x_dev), n_tokens, d, ldx, h_dev, ldh, alpha, beta, st);
 }
 

@@ -35,6 +35,8 @@ struct GemmArgs {
   // sweep kernel computes the ones it pulls), 2 also for K = 128 (the
   // blocked Cholesky's inner updates)
   int x6;
+  // device word (NULL: none): the general kernel does nothing where it is zero
+  const int* only_if;
 };
 
 // Whether products asking for x6 take it (MI355Q_GEMM_X6=0 turns it off).
@@ -46,8 +48,8 @@ int gemm_f32(const GemmArgs& g, bool b_trans, int batch, hipStream_t stream);
 
 // H[i][j] = beta * H[i][j] + alpha * sum_t x[t][i] x[t][j] for i <= j, x
 // [n, d] fp32 row-major (ldx): the fp32 MFMA product of the general kernel
-// with A = x transposed, upper tiles only.
+// with A = x transposed, upper tiles only.  only_if: as GemmArgs.
 int syrk_f32_upper(const float* x, int64_t n, int64_t d, int64_t ldx, float* h, int64_t ldh, float alpha,
-                   float beta, hipStream_t stream);
+                   float beta, hipStream_t stream, const int* only_if = nullptr);
 
 }  // namespace mi355q

@@ -45,6 +45,7 @@ __global__ __launch_bounds__(GNT, 2) void gemm_f32_kernel(GemmArgs g) {
   const int64_t m0 = (int64_t)blockIdx.y * GBM, n0 = (int64_t)blockIdx.x * GBN;
   if (g.lower_only && m0 + GBM - 1 < n0) return;
   if (g.upper_only && m0 > n0 + GBN - 1) return;
+  if (g.only_if && *g.only_if == 0) return;
   const int64_t bz = blockIdx.z;
   const int64_t b1 = g.inner > 0 ? bz % g.inner : bz, b2 = g.inner > 0 ? bz / g.inner : 0;
   const float* A = g.A + b1 * g.strideA + b2 * g.strideA2;
@@ -2297,8 +2298,9 @@ int gemm_f32(const GemmArgs& g, bool b_trans, int batch, hipStream_t stream) {
 }
 
 int syrk_f32_upper(const float* x, int64_t n, int64_t d, int64_t ldx, float* h, int64_t ldh, float alpha,
-                   float beta, hipStream_t stream) {
+                   float beta, hipStream_t stream, const int* only_if) {
   GemmArgs g{};
+  g.only_if = only_if;
   g.A = x; g.lda = ldx; g.a_trans = 1;
   g.B = x; g.ldb = ldx;
   g.C = h; g.ldc = ldh;

@@ -53,8 +53,9 @@ def hessian_syrk_(H: torch.Tensor, x: torch.Tensor, alpha: float = 2.0, beta: fl
     place (beta == 1: H += ...).
 
     ``x`` is [tokens, d] (row stride may exceed d) bf16 or fp16 (16-bit MFMA,
-    exact products) or fp32 (fp32 MFMA); other floating types are converted
-    to fp32.  H is fp32 [d, d].
+    exact products) or fp32 (six products of three bf16 planes, small ones on
+    the fp32 MFMA); other floating types are converted to fp32.  H is fp32
+    [d, d].
     """
     L.require_gpu(H, x)
     x = _hessian_input(x)
