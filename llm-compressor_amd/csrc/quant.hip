@@ -11,6 +11,7 @@
 #pragma clang fp contract(off)
 
 namespace mi355q {
+int64_t gemm_cus();  // compute units (the GEMM dispatch's count)
 namespace {
 
 constexpr int NT = 256;
@@ -294,7 +295,7 @@ __device__ __forceinline__ float shrink_p(int i, double grid) { return (float)(1
 // scales.
 template <bool B, bool ZP, bool IM, int FQ = 0>
 __device__ __forceinline__ float mse_term(float v, float s, float rs, float z, float qmin, float qmax, float norm,
-                                          const uint16_t* tab, float w) {
+                                          float w) {
   float t;
   if (B) {
     const float q0 = v * rs;
@@ -307,9 +308,7 @@ __device__ __forceinline__ float mse_term(float v, float s, float rs, float z, f
   t = FQ == 1 ? fp8e4m3_rne(t) : FQ >= 2 ? fp4e2m1_round(t) : rintf(t);
   if (ZP) t = rb<B>(t - z);
   if (IM) return pow_norm<false>(fabsf(rb<B>(t * s) - v), norm) * w;
-  const float d = fabsf(rb<B>(rb<B>(t * s) - v));
-  if (B) return __uint_as_float((uint32_t)tab[__float_as_uint(d) >> 16] << 16);
-  return pow_norm<false>(d, norm);
+  return pow_norm<false>(fabsf(t * s - v), norm);
 }
 
 // A candidate's scale and zero point from its shrunk min / max: CT
@@ -327,35 +326,140 @@ __device__ __forceinline__ void cand_qparams(const MseArgs& a, float mn, float m
   }
 }
 
+// two fp32 values to a packed bf16 pair (one v_cvt_pk_bf16_f32), first value
+// in the low half
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+  typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
+  typedef float f32x2v __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){a, b}, bf16x2v));
+}
+
+// Two terms at once.  bf16 values with the power table: the roundings go in
+// pairs (one v_cvt_pk_bf16_f32), and the errors' bits without their signs are
+// the table indexes.  med3 of a NaN is the smaller bound, as fmin(fmax())
+// gives.
+template <bool B, bool ZP, bool IM, int FQ>
+__device__ __forceinline__ void mse_terms(float v0, float v1, float s, float rs, float z, float qmin, float qmax,
+                                          float norm, const uint16_t* tab, float w0, float w1, float& e0, float& e1) {
+  if constexpr (B && !IM) {
+    auto round2 = [](float& x, float& y) __attribute__((always_inline)) {
+      const uint32_t p = pk_bf16(x, y);
+      x = __uint_as_float(p << 16);
+      y = __uint_as_float(p & 0xffff0000u);
+    };
+    const float q0 = v0 * rs, q1 = v1 * rs;
+    float t0 = fmaf(fmaf(-s, q0, v0), rs, q0), t1 = fmaf(fmaf(-s, q1, v1), rs, q1);
+    round2(t0, t1);
+    if (ZP) {
+      t0 += z;
+      t1 += z;
+      round2(t0, t1);
+    }
+    t0 = __builtin_amdgcn_fmed3f(t0, qmin, qmax);
+    t1 = __builtin_amdgcn_fmed3f(t1, qmin, qmax);
+    t0 = FQ == 1 ? fp8e4m3_rne(t0) : FQ >= 2 ? fp4e2m1_round(t0) : rintf(t0);
+    t1 = FQ == 1 ? fp8e4m3_rne(t1) : FQ >= 2 ? fp4e2m1_round(t1) : rintf(t1);
+    if (ZP) {
+      t0 -= z;
+      t1 -= z;
+      round2(t0, t1);
+    }
+    t0 *= s;
+    t1 *= s;
+    round2(t0, t1);
+    const uint32_t p = pk_bf16(t0 - v0, t1 - v1);
+    e0 = __uint_as_float((uint32_t)tab[p & 0x7fff] << 16);
+    e1 = __uint_as_float((uint32_t)tab[(p >> 16) & 0x7fff] << 16);
+  } else {
+    e0 = mse_term<B, ZP, IM, FQ>(v0, s, rs, z, qmin, qmax, norm, w0);
+    e1 = mse_term<B, ZP, IM, FQ>(v1, s, rs, z, qmin, qmax, norm, w1);
+  }
+}
+
+// A cell's first row and column, columns and values.  (64-bit division only
+// where the number of cells needs it: it costs over a hundred instructions.)
 __device__ __forceinline__ void cell_geom(const MseArgs& a, int64_t cell, int64_t& r0, int64_t& c0, int64_t& cwe,
                                           int64_t& n) {
-  const int64_t cr = cell / a.ncc, cq = cell % a.ncc;
+  int64_t cr, cq;
+  if (a.ncr * a.ncc < (int64_t(1) << 32)) {
+    cr = (uint32_t)cell / (uint32_t)a.ncc;
+    cq = (uint32_t)cell - (uint32_t)cr * (uint32_t)a.ncc;
+  } else {
+    cr = cell / a.ncc;
+    cq = cell % a.ncc;
+  }
   r0 = cr * a.ch;
   c0 = cq * a.cw;
   cwe = min(a.cw, a.cols - c0);
   n = cwe * min(a.ch, a.rows - r0);
 }
 
+// Value e of a cell (row-major): its offset from the cell's first value in
+// its row r and column c.
+__device__ __forceinline__ void cell_elem(const MseArgs& a, int64_t e, int64_t cwe, int64_t n, int64_t& r,
+                                          int64_t& c) {
+  if (a.ch == 1) {
+    r = 0;
+    c = e;
+  } else if (n < (int64_t(1) << 32)) {
+    r = (uint32_t)e / (uint32_t)cwe;
+    c = (uint32_t)e - (uint32_t)r * (uint32_t)cwe;
+  } else {
+    r = e / cwe;
+    c = e % cwe;
+  }
+}
+
 template <bool B>
 __device__ __forceinline__ void load_pow_table(uint16_t* tab, const uint16_t* table) {
   if (B) {
-    for (int i = threadIdx.x; i < POW_TAB / 8; i += NT)
+    for (int i = threadIdx.x; i < POW_TAB / 8; i += blockDim.x)
       reinterpret_cast<uint4*>(tab)[i] = reinterpret_cast<const uint4*>(table)[i];
     __syncthreads();
   }
 }
 
+// v + the v of another lane, by DPP control or by swapping row / wave halves
+template <int CTRL>
+__device__ __forceinline__ float add_dpp(float v) {
+  return v + __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float add_xor16(float v) {
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float add_xor32(float v) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+
+// The search is bound by its vector instructions: 16 a value and candidate
+// with integer codes and the table.  So what depends on the candidate alone
+// is computed once per cell, lane j holding candidate j's scale, and not in
+// every lane (with eight values a lane the scales cost as much as the
+// values); indexes are 32-bit where they fit, sums cross lanes by DPP, and
+// up to four 256-thread units share one workgroup's power table, so that
+// eight waves a SIMD fit beside a CU's two tables instead of two.  An
+// observer call on 4096 x 4096 bf16 in groups of 128 with 20 candidates takes
+// 187 us (428 with the table per 256 threads and the scales in every lane);
+// its instructions alone are about 130.
+constexpr int MSE_UNITS = 4;  // 256-thread units of a workgroup, at most
+
 // Cells of at most 8 * LG <= 512 values: LG lanes per cell, 8 values per
 // lane; workgroups loop over the cells (the table is loaded once each).
 template <bool B, bool ZP, bool IM, int FQ = 0>
-__global__ __launch_bounds__(NT) void mse_err_small_kernel(MseArgs a, int lg_log2, const uint16_t* table,
-                                                           float* err) {
+__global__ __launch_bounds__(MSE_UNITS* NT, B && !IM ? 8 : 4) void mse_err_small_kernel(MseArgs a, int lg_log2,
+                                                                         const uint16_t* table, float* err) {
   constexpr bool TAB = B && !IM;
   __shared__ uint16_t tab[TAB ? POW_TAB : 8];
   load_pow_table<TAB>(tab, table);
-  const int LG = 1 << lg_log2, per_wg = NT >> lg_log2;
+  const int LG = 1 << lg_log2, per_wg = blockDim.x >> lg_log2;
   const int64_t ncells = a.ncr * a.ncc;
   const int l = threadIdx.x & (LG - 1);
+  const int first = 4 * (threadIdx.x & 63 & ~(LG - 1));  // lane 0 of the cell, as a ds_bpermute address
+  auto bcast = [](int addr, float v) __attribute__((always_inline)) {
+    return __uint_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_uint(v)));
+  };
   for (int64_t base = (int64_t)blockIdx.x * per_wg; base < ncells; base += (int64_t)gridDim.x * per_wg) {
     const int64_t cell_raw = base + (threadIdx.x >> lg_log2);
     const bool live = cell_raw < ncells;
@@ -368,39 +472,63 @@ __global__ __launch_bounds__(NT) void mse_err_small_kernel(MseArgs a, int lg_log
     for (int k = 0; k < 8; ++k) {
       const int64_t e = l + (int64_t)k * LG;
       ok[k] = e < n;
-      const int64_t ee = ok[k] ? e : 0;
-      v[k] = load_elem(a.x, B ? MI355Q_BF16 : MI355Q_F32, (r0 + ee / cwe) * a.ldx + c0 + ee % cwe);
-      w[k] = (IM && a.imp) ? a.imp[c0 + ee % cwe] : 1.f;
+      int64_t r, c;
+      cell_elem(a, ok[k] ? e : 0, cwe, n, r, c);
+      v[k] = load_elem(a.x, B ? MI355Q_BF16 : MI355Q_F32, (r0 + r) * a.ldx + c0 + c);
+      w[k] = (IM && a.imp) ? a.imp[c0 + c] : 1.f;
     }
     const float mn = a.mn[cell], mx = a.mx[cell];
-    for (int i = 0; i < a.T; ++i) {
-      const float p = shrink_p(i, a.grid);
-      float s, z;
-      cand_qparams<B, ZP, FQ>(a, rb<B>(mn * p), rb<B>(mx * p), s, z);
-      const float rs = 1.f / s;
-      float acc = 0.f;
+    auto search = [&](auto full) __attribute__((always_inline)) {
+      for (int i0 = 0; i0 < a.T; i0 += LG) {
+        const int cnt = min(LG, a.T - i0);
+        const float p = shrink_p(min(i0 + l, a.T - 1), a.grid);
+        float sl, zl;
+        cand_qparams<B, ZP, FQ>(a, rb<B>(mn * p), rb<B>(mx * p), sl, zl);
+        const float rsl = 1.f / sl;
+        float mine = 0.f;
+        for (int j = 0; j < cnt; ++j) {
+          const float s = bcast(first + 4 * j, sl), rs = bcast(first + 4 * j, rsl);
+          const float z = ZP ? bcast(first + 4 * j, zl) : 0.f;
+          float acc = 0.f;
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        if (ok[k]) acc += mse_term<B, ZP, IM, FQ>(v[k], s, rs, z, a.qmin, a.qmax, a.norm, tab, w[k]);
-      for (int o = 1; o < LG; o <<= 1) acc += __shfl_xor(acc, o, LG);
-      if (live && l == 0) err[cell * a.T + i] = IM ? acc : rb<B>(acc);
-    }
+          for (int k = 0; k < 8; k += 2) {
+            float e0, e1;
+            mse_terms<B, ZP, IM, FQ>(v[k], v[k + 1], s, rs, z, a.qmin, a.qmax, a.norm, tab, w[k], w[k + 1], e0, e1);
+            if (decltype(full)::value || ok[k]) acc += e0;
+            if (decltype(full)::value || ok[k + 1]) acc += e1;
+          }
+          // lanes l ^ 1, 2, 4, .. in turn: each step's lanes hold equal sums
+          // within the groups of the steps before, so a mirror will do
+          if (lg_log2 > 0) acc = add_dpp<0xb1>(acc);    // quad_perm [1,0,3,2]
+          if (lg_log2 > 1) acc = add_dpp<0x4e>(acc);    // quad_perm [2,3,0,1]
+          if (lg_log2 > 2) acc = add_dpp<0x141>(acc);   // half-row mirror
+          if (lg_log2 > 3) acc = add_dpp<0x140>(acc);   // row mirror
+          if (lg_log2 > 4) acc = add_xor16(acc);
+          if (lg_log2 > 5) acc = add_xor32(acc);
+          if (l == j) mine = acc;
+        }
+        if (live && l < cnt) err[cell * a.T + i0 + l] = IM ? mine : rb<B>(mine);
+      }
+    };
+    if (__all(n == 8 * LG)) search(std::true_type{}); else search(std::false_type{});
   }
 }
 
 // Larger cells: chunks of 16 * NT values, one fp32 partial sum per chunk and
-// candidate (summed in chunk order by mse_flags_kernel); workgroups loop over
-// the (cell, chunk) items.
+// candidate (summed in chunk order by mse_flags_kernel); the workgroup's
+// 256-thread units loop over the (cell, chunk) items.
 template <bool B, bool ZP, bool IM, int FQ = 0>
-__global__ __launch_bounds__(NT) void mse_err_large_kernel(MseArgs a, int64_t nchunk, const uint16_t* table,
-                                                           float* part) {
+__global__ __launch_bounds__(MSE_UNITS* NT, B && !IM ? 8 : 4) void mse_err_large_kernel(MseArgs a, int64_t nchunk,
+                                                                         const uint16_t* table, float* part) {
   constexpr bool TAB = B && !IM;
   __shared__ uint16_t tab[TAB ? POW_TAB : 8];
-  __shared__ float red[NT / 64];
+  __shared__ float red[MSE_UNITS][NT / 64][64];
   load_pow_table<TAB>(tab, table);
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x % NT, lane = tid & 63, unit = threadIdx.x / NT, units = blockDim.x / NT;
   const int64_t nitems = a.ncr * a.ncc * nchunk;
-  for (int64_t item = blockIdx.x; item < nitems; item += gridDim.x) {
+  for (int64_t base = (int64_t)blockIdx.x * units; base < nitems; base += (int64_t)gridDim.x * units) {
+    const bool live = base + unit < nitems;
+    const int64_t item = live ? base + unit : nitems - 1;
     const int64_t cell = item / nchunk, chunk = item % nchunk;
     int64_t r0, c0, cwe, n;
     cell_geom(a, cell, r0, c0, cwe, n);
@@ -410,24 +538,48 @@ __global__ __launch_bounds__(NT) void mse_err_large_kernel(MseArgs a, int64_t nc
     for (int k = 0; k < 16; ++k) {
       const int64_t e = chunk * (16 * NT) + (int64_t)k * NT + tid;
       ok[k] = e < n;
-      const int64_t ee = ok[k] ? e : 0;
-      v[k] = load_elem(a.x, B ? MI355Q_BF16 : MI355Q_F32, (r0 + ee / cwe) * a.ldx + c0 + ee % cwe);
-      w[k] = (IM && a.imp) ? a.imp[c0 + ee % cwe] : 1.f;
+      int64_t r, c;
+      cell_elem(a, ok[k] ? e : 0, cwe, n, r, c);
+      v[k] = load_elem(a.x, B ? MI355Q_BF16 : MI355Q_F32, (r0 + r) * a.ldx + c0 + c);
+      w[k] = (IM && a.imp) ? a.imp[c0 + c] : 1.f;
     }
     const float mn = a.mn[cell], mx = a.mx[cell];
-    for (int i = 0; i < a.T; ++i) {
-      const float p = shrink_p(i, a.grid);
-      float s, z;
-      cand_qparams<B, ZP, FQ>(a, rb<B>(mn * p), rb<B>(mx * p), s, z);
-      const float rs = 1.f / s;
-      float acc = 0.f;
+    const bool whole = (chunk + 1) * (16 * NT) <= n;
+    for (int i0 = 0; i0 < a.T; i0 += 64) {
+      const int cnt = min(64, a.T - i0);
+      const float p = shrink_p(min(i0 + lane, a.T - 1), a.grid);
+      float sl, zl;
+      cand_qparams<B, ZP, FQ>(a, rb<B>(mn * p), rb<B>(mx * p), sl, zl);
+      const float rsl = 1.f / sl;
+      auto lane_of = [](float x, int j) __attribute__((always_inline)) {
+        return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), j));
+      };
+      auto search = [&](auto full) __attribute__((always_inline)) {
+        for (int j = 0; j < cnt; ++j) {
+          const float s = lane_of(sl, j), rs = lane_of(rsl, j), z = ZP ? lane_of(zl, j) : 0.f;
+          float acc = 0.f;
 #pragma unroll
-      for (int k = 0; k < 16; ++k)
-        if (ok[k]) acc += mse_term<B, ZP, IM, FQ>(v[k], s, rs, z, a.qmin, a.qmax, a.norm, tab, w[k]);
-      for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-      if ((tid & 63) == 0) red[tid >> 6] = acc;
+          for (int k = 0; k < 16; k += 2) {
+            float e0, e1;
+            mse_terms<B, ZP, IM, FQ>(v[k], v[k + 1], s, rs, z, a.qmin, a.qmax, a.norm, tab, w[k], w[k + 1], e0, e1);
+            if (decltype(full)::value || ok[k]) acc += e0;
+            if (decltype(full)::value || ok[k + 1]) acc += e1;
+          }
+          // lanes l ^ 32, 16, 8, .. in turn: each step's sums repeat with
+          // its distance, so rotations within the row will do
+          acc = add_xor16(add_xor32(acc));
+          acc = add_dpp<0x128>(acc);  // row rotations by 8, 4, 2, 1
+          acc = add_dpp<0x124>(acc);
+          acc = add_dpp<0x122>(acc);
+          acc = add_dpp<0x121>(acc);
+          if (lane == 0) red[unit][tid >> 6][j] = acc;
+        }
+      };
+      if (whole) search(std::true_type{}); else search(std::false_type{});
       __syncthreads();
-      if (tid == 0) part[(cell * nchunk + chunk) * a.T + i] = ((red[0] + red[1]) + red[2]) + red[3];
+      if (live && tid < cnt)
+        part[(cell * nchunk + chunk) * a.T + i0 + tid] =
+            ((red[unit][0][tid] + red[unit][1][tid]) + red[unit][2][tid]) + red[unit][3][tid];
       __syncthreads();
     }
   }
@@ -1083,7 +1235,13 @@ int observe_mse_impl(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_
     hipLaunchKernelGGL(mse_pow_table_kernel, dim3(POW_TAB / NT), dim3(NT), 0, st, norm, tab);
     MQ_LAUNCH_CHECK();
   }
-  constexpr int64_t kMaxWg = 1024;  // persistent workgroups (each loads the power table once)
+  // Persistent workgroups, each of which loads the power table once.  As many
+  // 256-thread units share one as leave no CU without a workgroup; two
+  // workgroups of four units fill a CU's 32 waves.
+  const int64_t work = pl.lg_log2 >= 0 ? (((ncells << pl.lg_log2) + NT - 1) / NT) : ncells * pl.nchunk;
+  const int64_t units = min(max(work / gemm_cus(), (int64_t)1), (int64_t)MSE_UNITS);
+  const dim3 g((unsigned)min((work + units - 1) / units, 2 * gemm_cus() * MSE_UNITS / units));
+  const dim3 nt((unsigned)(units * NT));
   // kernel variant for (bf16, zero points, imatrix mode)
   // (the float grids: symmetric only; f00 .. f11 (fp8) and h00 .. h11 (fp4)
   // are their (bf16, imatrix) variants)
@@ -1103,8 +1261,6 @@ int observe_mse_impl(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_
     }
   };
   if (pl.lg_log2 >= 0) {
-    const int64_t per_wg = NT >> pl.lg_log2;
-    const dim3 g((unsigned)min((ncells + per_wg - 1) / per_wg, kMaxWg));
     pick(mse_err_small_kernel<false, false, false>, mse_err_small_kernel<false, false, true>,
          mse_err_small_kernel<false, true, false>, mse_err_small_kernel<false, true, true>,
          mse_err_small_kernel<true, false, false>, mse_err_small_kernel<true, false, true>,
@@ -1115,9 +1271,8 @@ int observe_mse_impl(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_
          mse_err_small_kernel<true, false, false, 2>, mse_err_small_kernel<true, false, true, 2>,
          mse_err_small_kernel<false, false, false, 3>, mse_err_small_kernel<false, false, true, 3>,
          mse_err_small_kernel<true, false, false, 3>, mse_err_small_kernel<true, false, true, 3>,
-         [&](auto kernel) { hipLaunchKernelGGL(kernel, g, dim3(NT), 0, st, a, pl.lg_log2, tab, err); });
+         [&](auto kernel) { hipLaunchKernelGGL(kernel, g, nt, 0, st, a, pl.lg_log2, tab, err); });
   } else {
-    const dim3 g((unsigned)min(ncells * pl.nchunk, kMaxWg));
     pick(mse_err_large_kernel<false, false, false>, mse_err_large_kernel<false, false, true>,
          mse_err_large_kernel<false, true, false>, mse_err_large_kernel<false, true, true>,
          mse_err_large_kernel<true, false, false>, mse_err_large_kernel<true, false, true>,
@@ -1128,7 +1283,7 @@ int observe_mse_impl(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_
          mse_err_large_kernel<true, false, false, 2>, mse_err_large_kernel<true, false, true, 2>,
          mse_err_large_kernel<false, false, false, 3>, mse_err_large_kernel<false, false, true, 3>,
          mse_err_large_kernel<true, false, false, 3>, mse_err_large_kernel<true, false, true, 3>,
-         [&](auto kernel) { hipLaunchKernelGGL(kernel, g, dim3(NT), 0, st, a, pl.nchunk, tab, part); });
+         [&](auto kernel) { hipLaunchKernelGGL(kernel, g, nt, 0, st, a, pl.nchunk, tab, part); });
   }
   MQ_LAUNCH_CHECK();
   const bool round_sum = b && !im;
