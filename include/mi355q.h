@@ -335,6 +335,13 @@ int mi355q_observe_minmax(const void* x_dev, mi355q_dtype dtype, int64_t rows, i
                           int64_t ldx, int strategy, int64_t group_size, int block_h, int block_w,
                           float* min_dev, float* max_dev, void* stream);
 
+/* The same with the statistics in out_dtype: fp32, or bf16 those of bf16
+ * values (exact), any strategy but MI355Q_TENSOR. */
+int mi355q_observe_minmax_typed(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_t cols,
+                                int64_t ldx, int strategy, int64_t group_size, int block_h,
+                                int block_w, void* min_dev, void* max_dev, mi355q_dtype out_dtype,
+                                void* stream);
+
 /* CT calculate_qparams (observers/base.py:99-123 -> CT) over the quantized
  * range [qmin, qmax] ((-2^(b-1), 2^(b-1)-1) for int, (-448, 448) for fp8):
  * symmetric scale = absmax / ((qmax - qmin) / 2), asymmetric scale =
@@ -347,6 +354,14 @@ int mi355q_observe_minmax(const void* x_dev, mi355q_dtype dtype, int64_t rows, i
 int mi355q_calculate_qparams(const float* min_dev, const float* max_dev, int64_t n, float qmin,
                              float qmax, int symmetric, int strict, mi355q_dtype scale_dtype,
                              float* scale_out_dev, float* zp_out_dev, void* stream);
+
+/* The same from statistics of stats_dtype, with scales stored as
+ * scale_out_dtype (bf16 or fp32) and zero points as int8 or fp32. */
+int mi355q_calculate_qparams_typed(const void* min_dev, const void* max_dev, mi355q_dtype stats_dtype,
+                                   int64_t n, float qmin, float qmax, int symmetric, int strict,
+                                   mi355q_dtype scale_dtype, void* scale_out_dev,
+                                   mi355q_dtype scale_out_dtype, void* zp_out_dev, int zp_int8,
+                                   void* stream);
 
 /* MX shared scales from observer statistics: e8m0 byte per group (rule as
  * in mi355q_mxfp4_quantize_pack, absmax = max(|min|, |max|) of bf16
@@ -425,6 +440,14 @@ int mi355q_quantize_int(const void* x_dev, mi355q_dtype dtype, int64_t rows, int
                         int64_t ld_scale, const int32_t* g_idx_dev, int strategy,
                         int64_t group_size, int block_h, int block_w, int num_bits,
                         mi355q_dtype div_dtype, int8_t* codes_dev, void* stream);
+
+/* The same with bf16 or fp32 scales and int8 or fp32 zero points. */
+int mi355q_quantize_int_typed(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_t cols,
+                              int64_t ldx, const void* scale_dev, mi355q_dtype scale_dtype,
+                              const void* zp_dev, int zp_int8, int64_t ld_scale,
+                              const int32_t* g_idx_dev, int strategy, int64_t group_size, int block_h,
+                              int block_w, int num_bits, mi355q_dtype div_dtype, int8_t* codes_dev,
+                              void* stream);
 
 /* CT pack_quantized (pack_to_int32): 4-bit codes -> int32 words, eight per
  * word, element k of a word at bits 4k, stored offset-binary (q + 8).

@@ -22,6 +22,19 @@ __device__ __forceinline__ float load_elem(const void* x, mi355q_dtype dt, int64
                            : static_cast<const float*>(x)[i];
 }
 
+// Element i of a small operand that may be bf16 (statistics, scales) and its store
+__device__ __forceinline__ float load_stat(const void* p, bool b16, int64_t i) {
+  return b16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(p)[i]) : static_cast<const float*>(p)[i];
+}
+__device__ __forceinline__ void store_stat(void* p, bool b16, int64_t i, float v) {
+  if (b16) static_cast<uint16_t*>(p)[i] = f32_to_bf16_bits(v);
+  else static_cast<float*>(p)[i] = v;
+}
+// Zero points: int8 or fp32
+__device__ __forceinline__ float load_zp(const void* p, bool i8, int64_t i) {
+  return i8 ? (float)static_cast<const int8_t*>(p)[i] : static_cast<const float*>(p)[i];
+}
+
 // Total order on floats as signed ints, for atomic min/max.
 __device__ __forceinline__ int f2ord(float f) {
   int i = __float_as_int(f);
@@ -58,7 +71,7 @@ __device__ __forceinline__ int64_t scale_index(int strategy, int64_t r, int64_t 
 // One workgroup per row (CHANNEL / TOKEN) or the whole tensor (TENSOR, via
 // ordered-int atomics on pre-initialised outputs).
 __global__ void minmax_rows_kernel(const void* x, mi355q_dtype dt, int64_t rows, int64_t cols,
-                                   int64_t ldx, float* mn_out, float* mx_out, int tensor_mode) {
+                                   int64_t ldx, void* mn_out, void* mx_out, int out_b16, int tensor_mode) {
   __shared__ float smn[NT / 64], smx[NT / 64];
   const int64_t r = blockIdx.x;
   if (r >= rows) return;
@@ -100,8 +113,8 @@ __global__ void minmax_rows_kernel(const void* x, mi355q_dtype dt, int64_t rows,
       atomicMin(reinterpret_cast<int*>(mn_out), f2ord(mn));
       atomicMax(reinterpret_cast<int*>(mx_out), f2ord(mx));
     } else {
-      mn_out[r] = mn;
-      mx_out[r] = mx;
+      store_stat(mn_out, out_b16, r, mn);
+      store_stat(mx_out, out_b16, r, mx);
     }
   }
 }
@@ -118,7 +131,7 @@ __global__ void minmax_finish_kernel(float* mn, float* mx) {
 // Groups along columns, vector path: LPG lanes x 8 elements per group.
 template <int LPG>
 __global__ void minmax_group_vec_kernel(const uint16_t* x, int64_t rows, int64_t cols, int64_t ldx,
-                                        float* mn_out, float* mx_out) {
+                                        void* mn_out, void* mx_out, int out_b16) {
   const int64_t chunks_per_row = cols / 8;
   const int64_t total = rows * chunks_per_row;
   const int64_t ngroups = cols / (8 * LPG);
@@ -143,8 +156,8 @@ __global__ void minmax_group_vec_kernel(const uint16_t* x, int64_t rows, int64_t
     if (c < total && (threadIdx.x & (LPG - 1)) == 0) {
       const int64_t r = c / chunks_per_row, k = c % chunks_per_row;
       const int64_t g = k / LPG;
-      mn_out[r * ngroups + g] = mn;
-      mx_out[r * ngroups + g] = mx;
+      store_stat(mn_out, out_b16, r * ngroups + g, mn);
+      store_stat(mx_out, out_b16, r * ngroups + g, mx);
     }
   }
 }
@@ -152,7 +165,7 @@ __global__ void minmax_group_vec_kernel(const uint16_t* x, int64_t rows, int64_t
 // Generic groups / blocks: one thread per output cell, zero padding counted.
 __global__ void minmax_cells_kernel(const void* x, mi355q_dtype dt, int64_t rows, int64_t cols,
                                     int64_t ldx, int64_t cell_h, int64_t cell_w, int64_t ncr,
-                                    int64_t ncc, float* mn_out, float* mx_out) {
+                                    int64_t ncc, void* mn_out, void* mx_out, int out_b16) {
   const int64_t cell = (int64_t)blockIdx.x * NT + threadIdx.x;
   if (cell >= ncr * ncc) return;
   const int64_t cr = cell / ncc, cc = cell % ncc;
@@ -166,8 +179,8 @@ __global__ void minmax_cells_kernel(const void* x, mi355q_dtype dt, int64_t rows
       mx = fmaxf(mx, v);
     }
   }
-  mn_out[cell] = mn;
-  mx_out[cell] = mx;
+  store_stat(mn_out, out_b16, cell, mn);
+  store_stat(mx_out, out_b16, cell, mx);
 }
 
 // ---------------------------------------------------------------- qparams
@@ -196,15 +209,17 @@ __device__ __forceinline__ void qparams_one(float mn, float mx, float qmin, floa
   if (!strict && scale == 0.f) scale = b ? 0.0078125f : 1.1920928955078125e-07f;
 }
 
-__global__ void qparams_kernel(const float* mn_in, const float* mx_in, int64_t n, float qmin, float qmax,
-                               int symmetric, int strict, int bf16_scale, float* scale_out,
-                               float* zp_out) {
+__global__ void qparams_kernel(const void* mn_in, const void* mx_in, int in_b16, int64_t n, float qmin, float qmax,
+                               int symmetric, int strict, int bf16_scale, void* scale_out, int scale_b16,
+                               void* zp_out, int zp_i8) {
   const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
   if (i >= n) return;
   float scale, zp;
-  qparams_one(mn_in[i], mx_in[i], qmin, qmax, symmetric != 0, strict != 0, bf16_scale != 0, scale, zp);
-  scale_out[i] = scale;
-  zp_out[i] = zp;
+  qparams_one(load_stat(mn_in, in_b16, i), load_stat(mx_in, in_b16, i), qmin, qmax, symmetric != 0, strict != 0,
+              bf16_scale != 0, scale, zp);
+  store_stat(scale_out, scale_b16, i, scale);
+  if (zp_i8) static_cast<int8_t*>(zp_out)[i] = (int8_t)zp;
+  else static_cast<float*>(zp_out)[i] = zp;
 }
 
 // e8m0 exponent byte of an MX group scale from the group absmax (rule:
@@ -685,7 +700,7 @@ MsePlan plan_mse(int64_t rows, int64_t cols, int64_t ch, int64_t cw, int T) {
 
 // ---------------------------------------------------------------- int quantize
 __global__ void quantize_int_kernel(const void* x, mi355q_dtype dt, int64_t rows, int64_t cols,
-                                    int64_t ldx, const float* scale, const float* zp,
+                                    int64_t ldx, const void* scale, int scale_b16, const void* zp, int zp_i8,
                                     int64_t ld_scale, const int32_t* g_idx, int strategy,
                                     int64_t group_size, int bh, int bw, float qmin, float qmax,
                                     int div_bf16, int8_t* out) {
@@ -694,15 +709,62 @@ __global__ void quantize_int_kernel(const void* x, mi355q_dtype dt, int64_t rows
     const int64_t r = i / cols, c = i % cols;
     const int64_t si = scale_index(strategy, r, c, ld_scale, g_idx, group_size, bh, bw);
     float v = load_elem(x, dt, r * ldx + c);
-    float q = v / scale[si];
+    float q = v / load_stat(scale, scale_b16, si);
     if (div_bf16) q = round_to_bf16(q);
     if (zp) {
-      q = q + zp[si];
+      q = q + load_zp(zp, zp_i8, si);
       if (div_bf16) q = round_to_bf16(q);
     }
     q = fminf(fmaxf(q, qmin), qmax);
     out[r * cols + c] = (int8_t)rintf(q);
   }
+}
+
+// The same for rows of whole, 16-byte aligned chunks of 8 values that share
+// one scale (per tensor, row, or groups of a multiple of 8 columns): one chunk
+// a thread, 32-bit indexes (rows * cols < 2^32).  The 64-bit divisions of an
+// index cost the general kernel more than its values: 1024 x 4096 bf16 in
+// groups of 128 takes 5.9 us (15 there), of which the launch is about half.
+template <bool B>
+__global__ void quantize_int_vec_kernel(const void* x, uint32_t rows, uint32_t cols, int64_t ldx, const void* scale,
+                                        int scale_b16, const void* zp, int zp_i8, int64_t ld_scale, uint32_t group,
+                                        float qmin, float qmax, int div_bf16, int8_t* out) {
+  const uint32_t cpr = cols / 8, i = blockIdx.x * NT + threadIdx.x;
+  const uint32_t r = i / cpr, c = 8 * (i - r * cpr);
+  if (r >= rows) return;
+  float v[8];
+  if (B) {
+    const u32x4_t t = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(x) + r * ldx + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[2 * e] = __uint_as_float(t[e] << 16);
+      v[2 * e + 1] = __uint_as_float(t[e] & 0xffff0000u);
+    }
+  } else {
+    const f32x4_t* p = reinterpret_cast<const f32x4_t*>(static_cast<const float*>(x) + r * ldx + c);
+    const f32x4_t t0 = p[0], t1 = p[1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = t0[e];
+      v[4 + e] = t1[e];
+    }
+  }
+  // group 0: one scale per row (ld_scale 0: one for all)
+  const int64_t si = (int64_t)r * ld_scale + (group ? c / group : 0);
+  const float s = load_stat(scale, scale_b16, si), z = zp ? load_zp(zp, zp_i8, si) : 0.f;
+  uint32_t w[2] = {0, 0};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float q = v[e] / s;
+    if (div_bf16) q = round_to_bf16(q);
+    if (zp) {
+      q = q + z;
+      if (div_bf16) q = round_to_bf16(q);
+    }
+    q = fminf(fmaxf(q, qmin), qmax);
+    w[e / 4] |= ((uint32_t)(int)rintf(q) & 0xffu) << (8 * (e % 4));
+  }
+  *reinterpret_cast<uint2*>(out + (int64_t)r * cols + c) = make_uint2(w[0], w[1]);
 }
 
 // ---------------------------------------------------------------- packs
@@ -1108,24 +1170,29 @@ inline unsigned grid_for(int64_t n, int64_t per_block = NT, unsigned cap = 65536
 
 using namespace mi355q;
 
-extern "C" int mi355q_observe_minmax(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_t cols,
-                                     int64_t ldx, int strategy, int64_t group_size, int block_h,
-                                     int block_w, float* min_dev, float* max_dev, void* stream) {
+extern "C" int mi355q_observe_minmax_typed(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_t cols,
+                                           int64_t ldx, int strategy, int64_t group_size, int block_h, int block_w,
+                                           void* min_dev, void* max_dev, mi355q_dtype out_dtype, void* stream) {
   MQ_CHECK_ARG(x_dev && min_dev && max_dev, "observe_minmax: null pointer");
   MQ_CHECK_ARG(rows > 0 && cols > 0 && ldx >= cols, "observe_minmax: bad shape");
   MQ_CHECK_ARG(dtype == MI355Q_BF16 || dtype == MI355Q_F32, "observe_minmax: bad dtype");
+  MQ_CHECK_ARG(out_dtype == MI355Q_F32 || (out_dtype == MI355Q_BF16 && dtype == MI355Q_BF16 && strategy != MI355Q_TENSOR),
+               "observe_minmax: statistics are fp32, or bf16 those of bf16 values, not per tensor");
+  const int b16 = out_dtype == MI355Q_BF16 ? 1 : 0;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   switch (strategy) {
     case MI355Q_TENSOR:
-      hipLaunchKernelGGL(minmax_init_kernel, dim3(1), dim3(1), 0, st, min_dev, max_dev);
+      hipLaunchKernelGGL(minmax_init_kernel, dim3(1), dim3(1), 0, st, static_cast<float*>(min_dev),
+                         static_cast<float*>(max_dev));
       hipLaunchKernelGGL(minmax_rows_kernel, dim3((unsigned)rows), dim3(NT), 0, st, x_dev, dtype, rows,
-                         cols, ldx, min_dev, max_dev, 1);
-      hipLaunchKernelGGL(minmax_finish_kernel, dim3(1), dim3(1), 0, st, min_dev, max_dev);
+                         cols, ldx, min_dev, max_dev, 0, 1);
+      hipLaunchKernelGGL(minmax_finish_kernel, dim3(1), dim3(1), 0, st, static_cast<float*>(min_dev),
+                         static_cast<float*>(max_dev));
       break;
     case MI355Q_CHANNEL:
     case MI355Q_TOKEN:
       hipLaunchKernelGGL(minmax_rows_kernel, dim3((unsigned)rows), dim3(NT), 0, st, x_dev, dtype, rows,
-                         cols, ldx, min_dev, max_dev, 0);
+                         cols, ldx, min_dev, max_dev, b16, 0);
       break;
     case MI355Q_GROUP: {
       MQ_CHECK_ARG(group_size > 0, "observe_minmax: group_size must be > 0");
@@ -1137,17 +1204,18 @@ extern "C" int mi355q_observe_minmax(const void* x_dev, mi355q_dtype dtype, int6
       const unsigned g = grid_for(chunks, NT, 1u << 20);
       const uint16_t* xb = static_cast<const uint16_t*>(x_dev);
       if (vec && group_size % 8 == 0 && lpg == 4)
-        hipLaunchKernelGGL(minmax_group_vec_kernel<4>, dim3(g), dim3(NT), 0, st, xb, rows, cols, ldx, min_dev, max_dev);
+        hipLaunchKernelGGL(minmax_group_vec_kernel<4>, dim3(g), dim3(NT), 0, st, xb, rows, cols, ldx, min_dev, max_dev, b16);
       else if (vec && group_size % 8 == 0 && lpg == 8)
-        hipLaunchKernelGGL(minmax_group_vec_kernel<8>, dim3(g), dim3(NT), 0, st, xb, rows, cols, ldx, min_dev, max_dev);
+        hipLaunchKernelGGL(minmax_group_vec_kernel<8>, dim3(g), dim3(NT), 0, st, xb, rows, cols, ldx, min_dev, max_dev, b16);
       else if (vec && group_size % 8 == 0 && lpg == 16)
-        hipLaunchKernelGGL(minmax_group_vec_kernel<16>, dim3(g), dim3(NT), 0, st, xb, rows, cols, ldx, min_dev, max_dev);
+        hipLaunchKernelGGL(minmax_group_vec_kernel<16>, dim3(g), dim3(NT), 0, st, xb, rows, cols, ldx, min_dev, max_dev, b16);
       else if (vec && group_size % 8 == 0 && lpg == 2)
-        hipLaunchKernelGGL(minmax_group_vec_kernel<2>, dim3(g), dim3(NT), 0, st, xb, rows, cols, ldx, min_dev, max_dev);
+        hipLaunchKernelGGL(minmax_group_vec_kernel<2>, dim3(g), dim3(NT), 0, st, xb, rows, cols, ldx, min_dev, max_dev, b16);
       else {
         const int64_t ng = cols / group_size;
         hipLaunchKernelGGL(minmax_cells_kernel, dim3(grid_for(rows * ng, NT, 1u << 30)), dim3(NT), 0, st,
-                           x_dev, dtype, rows, cols, ldx, (int64_t)1, group_size, rows, ng, min_dev, max_dev);
+                           x_dev, dtype, rows, cols, ldx, (int64_t)1, group_size, rows, ng, min_dev, max_dev,
+                           b16);
       }
       break;
     }
@@ -1156,7 +1224,7 @@ extern "C" int mi355q_observe_minmax(const void* x_dev, mi355q_dtype dtype, int6
       const int64_t ncr = (rows + block_h - 1) / block_h, ncc = (cols + block_w - 1) / block_w;
       hipLaunchKernelGGL(minmax_cells_kernel, dim3(grid_for(ncr * ncc, NT, 1u << 30)), dim3(NT), 0, st,
                          x_dev, dtype, rows, cols, ldx, (int64_t)block_h, (int64_t)block_w, ncr, ncc,
-                         min_dev, max_dev);
+                         min_dev, max_dev, b16);
       break;
     }
     default:
@@ -1167,19 +1235,40 @@ extern "C" int mi355q_observe_minmax(const void* x_dev, mi355q_dtype dtype, int6
   return MI355Q_OK;
 }
 
-extern "C" int mi355q_calculate_qparams(const float* min_dev, const float* max_dev, int64_t n, float qmin,
-                                        float qmax, int symmetric, int strict, mi355q_dtype scale_dtype,
-                                        float* scale_out_dev, float* zp_out_dev, void* stream) {
+extern "C" int mi355q_observe_minmax(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_t cols,
+                                     int64_t ldx, int strategy, int64_t group_size, int block_h,
+                                     int block_w, float* min_dev, float* max_dev, void* stream) {
+  return mi355q_observe_minmax_typed(x_dev, dtype, rows, cols, ldx, strategy, group_size, block_h, block_w, min_dev,
+                                     max_dev, MI355Q_F32, stream);
+}
+
+extern "C" int mi355q_calculate_qparams_typed(const void* min_dev, const void* max_dev, mi355q_dtype stats_dtype,
+                                              int64_t n, float qmin, float qmax, int symmetric, int strict,
+                                              mi355q_dtype scale_dtype, void* scale_out_dev,
+                                              mi355q_dtype scale_out_dtype, void* zp_out_dev, int zp_int8,
+                                              void* stream) {
   MQ_CHECK_ARG(min_dev && max_dev && scale_out_dev && zp_out_dev, "calculate_qparams: null pointer");
   MQ_CHECK_ARG(qmin < 0.f && qmax > 0.f, "calculate_qparams: range must straddle zero");
   MQ_CHECK_ARG(!strict || symmetric, "calculate_qparams: strict requires symmetric");
   MQ_CHECK_ARG(scale_dtype == MI355Q_BF16 || scale_dtype == MI355Q_F32, "calculate_qparams: scale dtype must be bf16 or fp32");
+  MQ_CHECK_ARG((stats_dtype == MI355Q_BF16 || stats_dtype == MI355Q_F32) &&
+                   (scale_out_dtype == MI355Q_BF16 || scale_out_dtype == MI355Q_F32),
+               "calculate_qparams: statistics and scales must be bf16 or fp32");
+  MQ_CHECK_ARG(!zp_int8 || (qmin >= -128.f && qmax <= 127.f), "calculate_qparams: zero points beyond int8");
   if (n <= 0) return MI355Q_OK;
   hipLaunchKernelGGL(qparams_kernel, dim3(grid_for(n, NT, 1u << 30)), dim3(NT), 0,
-                     reinterpret_cast<hipStream_t>(stream), min_dev, max_dev, n, qmin, qmax, symmetric,
-                     strict, scale_dtype == MI355Q_BF16 ? 1 : 0, scale_out_dev, zp_out_dev);
+                     reinterpret_cast<hipStream_t>(stream), min_dev, max_dev, stats_dtype == MI355Q_BF16 ? 1 : 0, n,
+                     qmin, qmax, symmetric, strict, scale_dtype == MI355Q_BF16 ? 1 : 0, scale_out_dev,
+                     scale_out_dtype == MI355Q_BF16 ? 1 : 0, zp_out_dev, zp_int8);
   MQ_LAUNCH_CHECK();
   return MI355Q_OK;
+}
+
+extern "C" int mi355q_calculate_qparams(const float* min_dev, const float* max_dev, int64_t n, float qmin,
+                                        float qmax, int symmetric, int strict, mi355q_dtype scale_dtype,
+                                        float* scale_out_dev, float* zp_out_dev, void* stream) {
+  return mi355q_calculate_qparams_typed(min_dev, max_dev, MI355Q_F32, n, qmin, qmax, symmetric, strict, scale_dtype,
+                                        scale_out_dev, MI355Q_F32, zp_out_dev, 0, stream);
 }
 
 extern "C" size_t mi355q_observe_mse_workspace_size(int64_t rows, int64_t cols, int64_t cell_rows,
@@ -1404,25 +1493,55 @@ extern "C" int mi355q_nvfp4_qparams(const float* min_dev, const float* max_dev, 
   return MI355Q_OK;
 }
 
+extern "C" int mi355q_quantize_int_typed(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_t cols,
+                                         int64_t ldx, const void* scale_dev, mi355q_dtype scale_dtype,
+                                         const void* zp_dev, int zp_int8, int64_t ld_scale, const int32_t* g_idx_dev,
+                                         int strategy, int64_t group_size, int block_h, int block_w, int num_bits,
+                                         mi355q_dtype div_dtype, int8_t* codes_dev, void* stream) {
+  MQ_CHECK_ARG(x_dev && scale_dev && codes_dev, "quantize_int: null pointer");
+  MQ_CHECK_ARG(rows > 0 && cols > 0 && ldx >= cols, "quantize_int: bad shape");
+  MQ_CHECK_ARG((dtype == MI355Q_BF16 || dtype == MI355Q_F32) && (div_dtype == MI355Q_BF16 || div_dtype == MI355Q_F32),
+               "quantize_int: dtypes must be bf16 or fp32");
+  MQ_CHECK_ARG(scale_dtype == MI355Q_BF16 || scale_dtype == MI355Q_F32, "quantize_int: scales must be bf16 or fp32");
+  const int sb = scale_dtype == MI355Q_BF16 ? 1 : 0;
+  MQ_CHECK_ARG(num_bits >= 2 && num_bits <= 8, "quantize_int: num_bits must be in [2, 8]");
+  MQ_CHECK_ARG(strategy != MI355Q_GROUP || group_size > 0 || g_idx_dev, "quantize_int: group_size");
+  MQ_CHECK_ARG(strategy != MI355Q_BLOCK || (block_h > 0 && block_w > 0), "quantize_int: block");
+  const float qmin = -(float)(1 << (num_bits - 1)), qmax = (float)((1 << (num_bits - 1)) - 1);
+  // whole aligned chunks with a scale each: the vector kernel
+  const bool b = dtype == MI355Q_BF16, per_row = strategy == MI355Q_CHANNEL || strategy == MI355Q_TOKEN;
+  const bool group = strategy == MI355Q_GROUP && !g_idx_dev && group_size % 8 == 0 && group_size <= cols;
+  if ((strategy == MI355Q_TENSOR || per_row || group) && cols % 8 == 0 && rows * cols < (int64_t(1) << 32) &&
+      ldx % (b ? 8 : 4) == 0 && aligned16(x_dev) && (reinterpret_cast<uintptr_t>(codes_dev) & 7) == 0) {
+    const dim3 g((unsigned)((rows * (cols / 8) + NT - 1) / NT));
+    const int64_t lds = strategy == MI355Q_TENSOR ? 0 : ld_scale;
+    const uint32_t gs = group ? (uint32_t)group_size : 0u;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (b)
+      hipLaunchKernelGGL(quantize_int_vec_kernel<true>, g, dim3(NT), 0, st, x_dev, (uint32_t)rows, (uint32_t)cols,
+                         ldx, scale_dev, sb, zp_dev, zp_int8, lds, gs, qmin, qmax, div_dtype == MI355Q_BF16 ? 1 : 0, codes_dev);
+    else
+      hipLaunchKernelGGL(quantize_int_vec_kernel<false>, g, dim3(NT), 0, st, x_dev, (uint32_t)rows, (uint32_t)cols,
+                         ldx, scale_dev, sb, zp_dev, zp_int8, lds, gs, qmin, qmax, div_dtype == MI355Q_BF16 ? 1 : 0, codes_dev);
+    MQ_LAUNCH_CHECK();
+    return MI355Q_OK;
+  }
+  hipLaunchKernelGGL(quantize_int_kernel, dim3(grid_for(rows * cols, NT, 1u << 16)), dim3(NT), 0,
+                     reinterpret_cast<hipStream_t>(stream), x_dev, dtype, rows, cols, ldx, scale_dev, sb,
+                     zp_dev, zp_int8, ld_scale, g_idx_dev, strategy, group_size, block_h, block_w, qmin, qmax,
+                     div_dtype == MI355Q_BF16 ? 1 : 0, codes_dev);
+  MQ_LAUNCH_CHECK();
+  return MI355Q_OK;
+}
+
 extern "C" int mi355q_quantize_int(const void* x_dev, mi355q_dtype dtype, int64_t rows, int64_t cols,
                                    int64_t ldx, const float* scale_dev, const float* zp_dev,
                                    int64_t ld_scale, const int32_t* g_idx_dev, int strategy,
                                    int64_t group_size, int block_h, int block_w, int num_bits,
                                    mi355q_dtype div_dtype, int8_t* codes_dev, void* stream) {
-  MQ_CHECK_ARG(x_dev && scale_dev && codes_dev, "quantize_int: null pointer");
-  MQ_CHECK_ARG(rows > 0 && cols > 0 && ldx >= cols, "quantize_int: bad shape");
-  MQ_CHECK_ARG((dtype == MI355Q_BF16 || dtype == MI355Q_F32) && (div_dtype == MI355Q_BF16 || div_dtype == MI355Q_F32),
-               "quantize_int: dtypes must be bf16 or fp32");
-  MQ_CHECK_ARG(num_bits >= 2 && num_bits <= 8, "quantize_int: num_bits must be in [2, 8]");
-  MQ_CHECK_ARG(strategy != MI355Q_GROUP || group_size > 0 || g_idx_dev, "quantize_int: group_size");
-  MQ_CHECK_ARG(strategy != MI355Q_BLOCK || (block_h > 0 && block_w > 0), "quantize_int: block");
-  const float qmin = -(float)(1 << (num_bits - 1)), qmax = (float)((1 << (num_bits - 1)) - 1);
-  hipLaunchKernelGGL(quantize_int_kernel, dim3(grid_for(rows * cols, NT, 1u << 16)), dim3(NT), 0,
-                     reinterpret_cast<hipStream_t>(stream), x_dev, dtype, rows, cols, ldx, scale_dev,
-                     zp_dev, ld_scale, g_idx_dev, strategy, group_size, block_h, block_w, qmin, qmax,
-                     div_dtype == MI355Q_BF16 ? 1 : 0, codes_dev);
-  MQ_LAUNCH_CHECK();
-  return MI355Q_OK;
+  return mi355q_quantize_int_typed(x_dev, dtype, rows, cols, ldx, scale_dev, MI355Q_F32, zp_dev, 0, ld_scale,
+                                   g_idx_dev, strategy, group_size, block_h, block_w, num_bits, div_dtype, codes_dev,
+                                   stream);
 }
 
 extern "C" int mi355q_pack_int4_int32(const int8_t* codes_dev, int64_t rows, int64_t cols,
@@ -1442,6 +1561,8 @@ extern "C" int mi355q_pack_int32(const int8_t* codes_dev, int64_t rows, int64_t 
   MQ_CHECK_ARG(rows > 0 && cols > 0, "pack_int32: bad shape");
   MQ_CHECK_ARG(num_bits == 2 || num_bits == 4 || num_bits == 8, "pack_int32: num_bits must be 2, 4 or 8");
   const int64_t wpr = (cols + 32 / num_bits - 1) / (32 / num_bits);
+  if (num_bits == 4 && cols % 8 == 0 && (reinterpret_cast<uintptr_t>(codes_dev) & 7) == 0)  // whole words: 8 codes a load
+    return mi355q_pack_int4_int32(codes_dev, rows, cols, out_dev, stream);
   hipLaunchKernelGGL(pack_int32_kernel, dim3(grid_for(rows * wpr, NT, 1u << 16)), dim3(NT), 0,
                      reinterpret_cast<hipStream_t>(stream), codes_dev, rows, cols, num_bits, wpr, out_dev);
   MQ_LAUNCH_CHECK();

@@ -61,6 +61,11 @@ SIGNATURES = {
     "mi355q_sparsegpt_workspace_size": (_sz, [_i64, _i64, _i64]),
     "mi355q_sparsegpt_sweep": (_i32, [_vp, _i64, _i64, _vp, _f64, _i32, _i32, _i64, _vp, _vp, _vp, _sz, _vp]),
     "mi355q_observe_minmax": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _i64, _i32, _i32, _vp, _vp, _vp]),
+    "mi355q_observe_minmax_typed": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _i64, _i32, _i32, _vp, _vp, _i32, _vp]),
+    "mi355q_calculate_qparams_typed": (_i32, [_vp, _vp, _i32, _i64, _f32, _f32, _i32, _i32, _i32, _vp, _i32, _vp, _i32,
+                                              _vp]),
+    "mi355q_quantize_int_typed": (_i32, [_vp, _i32, _i64, _i64, _i64, _vp, _i32, _vp, _i32, _i64, _vp, _i32, _i64,
+                                         _i32, _i32, _i32, _i32, _vp, _vp]),
     "mi355q_calculate_qparams": (_i32, [_vp, _vp, _i64, _f32, _f32, _i32, _i32, _i32, _vp, _vp, _vp]),
     "mi355q_observe_mse_workspace_size": (_sz, [_i64, _i64, _i64, _i64, _i32]),
     "mi355q_observe_mse": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _i32, _i32, _i32, _i32,
@@ -143,7 +148,14 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return t.data_ptr()
 
 
+# The current stream's handle without a Stream object around it: four calls of
+# the latter are an eighth of the host time of rounding a small weight.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(t.device.index)
     return torch.cuda.current_stream(t.device).cuda_stream
 
 

@@ -130,7 +130,7 @@ class Observer(torch.nn.Module):
         if self.is_weight_obs:
             if s == QuantizationStrategy.TOKEN:
                 raise ValueError("Token quantization cannot be applied to weights")
-            return ops.observe_minmax(observed, s.value, a.group_size, a.block_structure)
+            return ops.observe_minmax(observed, s.value, a.group_size, a.block_structure, dtype=observed.dtype)
         # activations: (batch, seq, hidden) -> rows = tokens
         x2 = observed.reshape(-1, observed.shape[-1])
         if s == QuantizationStrategy.TENSOR:
@@ -188,11 +188,12 @@ class Observer(torch.nn.Module):
             out = {"scale": scale, "zero_point": zp, "global_scale": gs}
         else:
             qmin, qmax = a.q_range()
-            scale, zp = ops.calculate_qparams(self.min_vals, self.max_vals, qmin, qmax, a.symmetric, dt)
             if a.type == QuantizationType.FLOAT and not a.symmetric:
                 raise NotImplementedError("asymmetric float quantization")
-            scale = scale.to(a.scale_dtype if a.scale_dtype is not None else dt)
-            out = {"scale": scale, "zero_point": zp.to(a.zp_dtype), "global_scale": None}
+            scale, zp = ops.calculate_qparams(self.min_vals, self.max_vals, qmin, qmax, a.symmetric, dt,
+                                              out_dtype=a.scale_dtype if a.scale_dtype is not None else dt,
+                                              zp_dtype=a.zp_dtype)
+            out = {"scale": scale, "zero_point": zp, "global_scale": None}
         self.delete_statistics()
         return out
 

@@ -370,8 +370,9 @@ def gptq_store_weight_batched(w_work: torch.Tensor, invperm, out_dtype: torch.dt
 
 # ---------------------------------------------------------------- observers
 def observe_minmax(x: torch.Tensor, strategy: str, group_size: int | None = None,
-                   block_structure=None):
-    """Min/max statistics of a 2-D tensor per strategy, as fp32 tensors.
+                   block_structure=None, dtype: torch.dtype = torch.float32):
+    """Min/max statistics of a 2-D tensor per strategy, as fp32 tensors or,
+    of a bf16 tensor, with ``dtype`` bf16.
 
     Shapes: tensor -> [1]; channel/token -> [rows, 1]; group ->
     [rows, cols / group]; block -> [ceil(rows/bh), ceil(cols/bw)].
@@ -396,26 +397,33 @@ def observe_minmax(x: torch.Tensor, strategy: str, group_size: int | None = None
         shape = (-(-rows // bh), -(-cols // bw))
     else:
         raise ValueError(f"unknown strategy {strategy}")
-    mn = torch.empty(shape, dtype=torch.float32, device=x.device)
-    mx = torch.empty(shape, dtype=torch.float32, device=x.device)
-    L.call("mi355q_observe_minmax", x.data_ptr(), _dt(x), rows, cols, x.stride(0), STRATEGY_CODE[strategy],
-           group_size or 0, bh, bw, mn.data_ptr(), mx.data_ptr(), L.stream_of(x))
-    return mn, mx
+    out = torch.bfloat16 if dtype == x.dtype == torch.bfloat16 and strategy != "tensor" else torch.float32
+    mn = torch.empty(shape, dtype=out, device=x.device)
+    mx = torch.empty(shape, dtype=out, device=x.device)
+    L.call("mi355q_observe_minmax_typed", x.data_ptr(), _dt(x), rows, cols, x.stride(0), STRATEGY_CODE[strategy],
+           group_size or 0, bh, bw, mn.data_ptr(), mx.data_ptr(), _dt(mn), L.stream_of(x))
+    return (mn, mx) if out == dtype else (mn.to(dtype), mx.to(dtype))
 
 
 def calculate_qparams(mn: torch.Tensor, mx: torch.Tensor, qmin: float, qmax: float, symmetric: bool,
-                      scale_dtype: torch.dtype, strict: bool = False):
-    """Scale / zero-point from min/max statistics (fp32 outputs holding
-    ``scale_dtype`` values and integer zero-points)."""
+                      scale_dtype: torch.dtype, strict: bool = False, out_dtype: torch.dtype = torch.float32,
+                      zp_dtype: torch.dtype = torch.float32):
+    """Scale / zero-point from min/max statistics (outputs holding
+    ``scale_dtype`` values, stored as ``out_dtype``, and integer zero-points,
+    stored as ``zp_dtype``)."""
     L.require_gpu(mn, mx)
-    mn = mn.to(torch.float32).contiguous()
-    mx = mx.to(torch.float32).contiguous()
-    scale = torch.empty_like(mn)
-    zp = torch.empty_like(mn)
-    L.call("mi355q_calculate_qparams", mn.data_ptr(), mx.data_ptr(), mn.numel(), C.c_float(qmin),
-           C.c_float(qmax), 1 if symmetric else 0, 1 if strict else 0,
-           L.BF16 if scale_dtype == torch.bfloat16 else L.F32, scale.data_ptr(), zp.data_ptr(), L.stream_of(mn))
-    return scale, zp
+    if mn.dtype != mx.dtype or mn.dtype != torch.bfloat16:
+        mn, mx = mn.to(torch.float32), mx.to(torch.float32)
+    mn, mx = mn.contiguous(), mx.contiguous()
+    # the kernel stores bf16 / fp32 scales and int8 / fp32 zero points
+    st = out_dtype if out_dtype in (torch.bfloat16, torch.float32) else torch.float32
+    zt = zp_dtype if zp_dtype == torch.int8 and qmin >= -128 and qmax <= 127 else torch.float32
+    scale = torch.empty_like(mn, dtype=st)
+    zp = torch.empty_like(mn, dtype=zt)
+    L.call("mi355q_calculate_qparams_typed", mn.data_ptr(), mx.data_ptr(), _dt(mn), mn.numel(), qmin, qmax,
+           1 if symmetric else 0, 1 if strict else 0, L.BF16 if scale_dtype == torch.bfloat16 else L.F32,
+           scale.data_ptr(), _dt(scale), zp.data_ptr(), 1 if zt == torch.int8 else 0, L.stream_of(mn))
+    return scale if st == out_dtype else scale.to(out_dtype), zp if zt == zp_dtype else zp.to(zp_dtype)
 
 
 MX_RULES = {"ct": L.MX_RULE_CT, "ocp": L.MX_RULE_OCP}
@@ -455,17 +463,19 @@ def quantize_int(x: torch.Tensor, scale: torch.Tensor, zero_point, strategy: str
     if x.stride(1) != 1:
         x = x.contiguous()
     rows, cols = x.shape
-    s = scale.to(torch.float32).contiguous()
+    s = (scale if scale.dtype == torch.bfloat16 else scale.to(torch.float32)).contiguous()
     s2 = s.reshape(-1, 1) if s.dim() < 2 else s
-    z = None if zero_point is None else \
-        zero_point.to(device=x.device, dtype=torch.float32).reshape(s2.shape).contiguous()
+    z = None
+    if zero_point is not None:
+        zt = torch.int8 if zero_point.dtype == torch.int8 else torch.float32
+        z = zero_point.to(device=x.device, dtype=zt).reshape(s2.shape).contiguous()
     gi = None if g_idx is None else g_idx.to(device=x.device, dtype=torch.int32).contiguous()
     bh, bw = block_structure if block_structure else (1, 1)
     if div_dtype is None:
         div_dtype = torch.promote_types(x.dtype, scale.dtype)
     out = torch.empty((rows, cols), dtype=torch.int8, device=x.device)
-    L.call("mi355q_quantize_int", x.data_ptr(), _dt(x), rows, cols, x.stride(0), s2.data_ptr(), L.ptr(z),
-           s2.stride(0), L.ptr(gi), STRATEGY_CODE[strategy], group_size or 0, bh, bw, num_bits,
+    L.call("mi355q_quantize_int_typed", x.data_ptr(), _dt(x), rows, cols, x.stride(0), s2.data_ptr(), _dt(s2),
+           L.ptr(z), 1 if z is not None and z.dtype == torch.int8 else 0, s2.stride(0), L.ptr(gi), STRATEGY_CODE[strategy], group_size or 0, bh, bw, num_bits,
            L.BF16 if div_dtype == torch.bfloat16 else L.F32, out.data_ptr(), L.stream_of(x))
     return out
 
