@@ -576,50 +576,7 @@ __device__ __forceinline__ void dma16(const void* gaddr, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gaddr), "s"(lds_addr) : "memory", "m0");
 }
 
-// fp32-accurate products on the bf16 MFMA ("x6"): every fp32 operand value
-// v is split exactly into three bf16 parts, v = h + m + l (h = bf16(v),
-// m = bf16(v - h), l = v - h - m, which has at most 8 significant bits and
-// is exact in bf16; the subtractions are exact in fp32), and a 16-deep slice
-// of A B is summed as the six products h h', h m', m h', h l', m m', l h'
-// on v_mfma_f32_32x32x16_bf16 (exact products, fp32 accumulation).  The
-// three dropped products are below 2^-24 of |a| |b| each, about the rounding
-// of one fp32 product; the sum is rounded in the MFMA's fp32 accumulator, as
-// on the fp32 MFMA.  Six bf16 MFMAs (192 cycles) replace the eight fp32
-// MFMAs (512 cycles) of a 16-deep slice; the splits (44 VALU instructions
-// per eight values, each wave splitting its own fragments) then bound the
-// kernel, since a wave's VALU work and its MFMAs were measured not to
-// overlap (busy cycles add up): the GPTQ lazy update 4096 x 3072 x 1024
-// takes 202 us against 248 us on the fp32 MFMA.  (Operands beyond 3.39e38,
-// where bf16 rounding overflows, do not occur in the solve's products.)
-
-// two fp32 values to a packed bf16 pair (one v_cvt_pk_bf16_f32, round to
-// nearest even), first value in the low half
-__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
-  typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
-  typedef float f32x2v __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){a, b}, bf16x2v));
-}
-// the exact three-part split of a pair: 11 VALU instructions (the bf16
-// halves read back as fp32 by a shift and a mask)
-__device__ __forceinline__ void split_x6_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-  h = pk_bf16(a, b);
-  const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
-  m = pk_bf16(ra, rb);
-  const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
-  l = pk_bf16(sa, sb);
-}
-__device__ __forceinline__ void split_x6(const f32x4_t& lo4, const f32x4_t& hi4, bf16x8_t* o) {
-  uint32_t h[4], m[4], l[4];
-  split_x6_pair(lo4[0], lo4[1], h[0], m[0], l[0]);
-  split_x6_pair(lo4[2], lo4[3], h[1], m[1], l[1]);
-  split_x6_pair(hi4[0], hi4[1], h[2], m[2], l[2]);
-  split_x6_pair(hi4[2], hi4[3], h[3], m[3], l[3]);
-  o[0] = __builtin_bit_cast(bf16x8_t, (u32x4_t){h[0], h[1], h[2], h[3]});
-  o[1] = __builtin_bit_cast(bf16x8_t, (u32x4_t){m[0], m[1], m[2], m[3]});
-  o[2] = __builtin_bit_cast(bf16x8_t, (u32x4_t){l[0], l[1], l[2], l[3]});
-}
-
-template <int TM, int TN, int WGM, int WGN, bool BT, int NS, bool X6 = false>
+template <int TM, int TN, int WGM, int WGN, bool BT, int NS>
 __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_dma_kernel(GemmArgs g) {
   constexpr int NW = WGM * WGN;
   constexpr int WTM = TM / WGM, WTN = TN / WGN;      // wave tile
@@ -773,84 +730,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_dma_kernel(GemmArgs g)
   };
 
   constexpr int ND = DA + DB;
-  if constexpr (X6) {
-    static_assert(NS >= 3 && (NS - 1) * ND < 64 && MB * NB2 > 1, "x6: three or more ring slots, two or more 32 x 32 blocks per wave");
-    // Per stage two 16-deep steps (groups 0, 1 and 2, 3).  The barrier that
-    // publishes stage st + 1 sits between them: the MFMAs of a step run
-    // interleaved with the splits of the next step's operands, also across
-    // the stage boundary, so the MFMA pipe is fed while the VALU splits.
-    struct Split { bf16x8_t a[MB][3], b[NB2][3]; };
-    auto split_step = [&](const Frag& fe, const Frag& fo, Split& sp) __attribute__((always_inline)) {
-#pragma unroll
-      for (int bm = 0; bm < MB; ++bm) split_x6(fe.a[bm], fo.a[bm], sp.a[bm]);
-#pragma unroll
-      for (int bn = 0; bn < NB2; ++bn) split_x6(fe.b[bn], fo.b[bn], sp.b[bn]);
-    };
-    // the six products per block, term-major so that consecutive MFMAs
-    // update different accumulators
-    auto mma_x6 = [&](const Split& sp) __attribute__((always_inline)) {
-      constexpr int TA[6] = {1, 2, 0, 1, 0, 0}, TB[6] = {1, 0, 2, 0, 1, 0};
-#pragma unroll
-      for (int t = 0; t < 6; ++t)
-#pragma unroll
-        for (int bm = 0; bm < MB; ++bm)
-#pragma unroll
-          for (int bn = 0; bn < NB2; ++bn)
-            acc[bm * NB2 + bn] =
-                __builtin_amdgcn_mfma_f32_32x32x16_bf16(sp.a[bm][TA[t]], sp.b[bn][TB[t]], acc[bm * NB2 + bn], 0, 0, 0);
-    };
-    // MFMAs of one step with the VALU work of the next step's split between
-    // them (44 VALU instructions per eight values split; a 32-cycle MFMA
-    // leaves room for about seven)
-    constexpr int VPM = (44 * (MB + NB2) + 6 * MB * NB2 - 1) / (6 * MB * NB2);
-    auto interleave = [&]() __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < 6 * MB * NB2; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
-      }
-    };
-    if (nst > 0) {
-#pragma unroll
-      for (int p = 0; p < NS; ++p)
-#pragma unroll
-        for (int i = 0; i < ND; ++i) issue(p, i);
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * ND) : "memory");
-      Split s0, s1;
-      {
-        Frag fe, fo;
-        read_group(lds, 0, fe);
-        read_group(lds, 1, fo);
-        split_step(fe, fo, s0);
-      }
-      for (int64_t st = 0; st < nst; ++st) {
-        const char* sl = lds + (st % NS) * SBYTES;
-        {
-          Frag fe, fo;
-          read_group(sl, 2, fe);
-          read_group(sl, 3, fo);
-          mma_x6(s0);
-          split_step(fe, fo, s1);
-          interleave();
-        }
-        // stage st + 1 complete (st + 2 may be in flight) and every wave
-        // done reading stage st, whose slot then takes stage st + 3
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * ND) : "memory");
-#pragma unroll
-        for (int i = 0; i < ND; ++i) issue(st + NS, i);
-        {
-          Frag fe, fo;
-          const char* sn = lds + ((st + 1) % NS) * SBYTES;
-          read_group(sn, 0, fe);
-          read_group(sn, 1, fo);
-          mma_x6(s1);
-          split_step(fe, fo, s0);   // past the last stage: a re-read of the last stage, never used
-          interleave();
-        }
-      }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-  } else if (nst > 0) {
+  if (nst > 0) {
 #pragma unroll
     for (int p = 0; p < NS - 1; ++p)
 #pragma unroll
@@ -909,6 +789,344 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_dma_kernel(GemmArgs g)
           if (!decltype(masked)::value || (gm < g.M && gn < g.N && (!g.lower_only || gm >= gn))) {
             const float sum = NBLK == 1 ? acc[0][r] + acc[1][r] : acc[bm * NB2 + bn][r];
             const float prod = g.alpha * sum;
+            g.C[gm * g.ldc + gn] = g.beta == 0.f ? prod : g.beta * cv[(bm * NB2 + bn) * 16 + r] + prod;
+          }
+        }
+  };
+  if (whole) put(std::false_type{}); else put(std::true_type{});
+}
+
+// fp32-accurate products on the bf16 MFMA ("x6"): every fp32 operand value
+// v is split exactly into three bf16 parts, v = h + m + l (h = bf16(v),
+// m = bf16(v - h), l = v - h - m, which has at most 8 significant bits and
+// is exact in bf16; the subtractions are exact in fp32), and a 16-deep slice
+// of A B is summed as the six products h h', h m', m h', h l', m m', l h'
+// on v_mfma_f32_32x32x16_bf16 (exact products, fp32 accumulation).  The
+// three dropped products are below 2^-24 of |a| |b| each, about the rounding
+// of one fp32 product; the sum is rounded in the MFMA's fp32 accumulator, as
+// on the fp32 MFMA.  Six bf16 MFMAs (192 cycles) replace the eight fp32
+// MFMAs (512 cycles) of a 16-deep slice.  (Operands beyond 3.39e38, where
+// bf16 rounding overflows, do not occur in the solve's products.)
+//
+// A split takes 44 VALU instructions per eight values: a wave that splits its
+// own operands, as many as its MFMAs take, spends as long on it.  So a
+// workgroup splits each value of its tile once: the threads load the fp32
+// values of a 32-deep stage into registers, split them and write the three
+// parts to LDS in 16-byte chunks of 8 k, ordered [part][k / 8][row], which
+// every wave reads as its MFMA operands.  How splits and MFMAs come to overlap
+// differs by tile:
+//   256 x 128  eight waves, two stages of parts: of the two waves on a SIMD one
+//              splits the next stage while the other multiplies this one
+//   128 x 128  four waves, one stage of parts; two workgroups on a CU, out of
+//              step by themselves
+//   64 x 128   four waves with a CU mostly to themselves: two stages, loads two
+//              stages ahead, each wave's splits scheduled between its MFMAs
+// Lazy updates of 4096 rows, K = 1024, against each wave splitting its own: N =
+// 3072 184 -> 131 us, N = 2048 103 -> 83 us; 14336 x 3072 663 -> 441 us; 64
+// products of 768 x 1536, K = 512, 514 -> 402 us; 256 x 3072 36 -> 30 us.  The
+// sums are the same bits: the same products in the same order.
+
+// two fp32 values to a packed bf16 pair (one v_cvt_pk_bf16_f32, round to
+// nearest even), first value in the low half
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+  typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
+  typedef float f32x2v __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){a, b}, bf16x2v));
+}
+// the exact three-part split of a pair: 11 VALU instructions (the bf16
+// halves read back as fp32 by a shift and a mask)
+__device__ __forceinline__ void split_x6_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = pk_bf16(a, b);
+  const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+  m = pk_bf16(ra, rb);
+  const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
+  l = pk_bf16(sa, sb);
+}
+__device__ __forceinline__ void split_x6(const f32x4_t& lo4, const f32x4_t& hi4, bf16x8_t* o) {
+  uint32_t h[4], m[4], l[4];
+  split_x6_pair(lo4[0], lo4[1], h[0], m[0], l[0]);
+  split_x6_pair(lo4[2], lo4[3], h[1], m[1], l[1]);
+  split_x6_pair(hi4[0], hi4[1], h[2], m[2], l[2]);
+  split_x6_pair(hi4[2], hi4[3], h[3], m[3], l[3]);
+  o[0] = __builtin_bit_cast(bf16x8_t, (u32x4_t){h[0], h[1], h[2], h[3]});
+  o[1] = __builtin_bit_cast(bf16x8_t, (u32x4_t){m[0], m[1], m[2], m[3]});
+  o[2] = __builtin_bit_cast(bf16x8_t, (u32x4_t){l[0], l[1], l[2], l[3]});
+}
+
+template <int TM, int TN, int WGM, int WGN, bool BT>
+__global__ __launch_bounds__(64 * WGM * WGN, 2) void gemm_x6_kernel(GemmArgs g) {
+  constexpr int NTH = 64 * WGM * WGN;
+  constexpr bool HALVES = NTH == 512, DEEP = TM == 64, DB = HALVES || DEEP;   // DB: two stages of parts
+  constexpr int WTM = TM / WGM, WTN = TN / WGN;       // wave tile
+  constexpr int MB = WTM / 32, NB2 = WTN / 32;
+  constexpr int UA = TM * 4 / NTH, UB = TN * 4 / NTH; // 8-value units of a thread and stage
+  static_assert(UA * NTH == TM * 4 && UB * NTH == TN * 4, "tile / thread split");
+  // bytes from one 8-deep chunk of all rows to the next: the 32 on top keep the
+  // four chunks of a row, written by neighbouring lanes, on different banks
+  constexpr int ASTR = TM * 16 + 32, BSTR = TN * 16 + 32;
+  constexpr int APL = 4 * ASTR, BPL = 4 * BSTR, BOFF = 3 * APL, STAGE = 3 * (APL + BPL);
+  __shared__ __attribute__((aligned(1024))) char lds[(DB ? 2 : 1) * STAGE];
+  {
+    const int64_t bz = blockIdx.z;
+    const int64_t b1 = g.inner > 0 ? bz % g.inner : bz, b2 = g.inner > 0 ? bz / g.inner : 0;
+    g.A += b1 * g.strideA + b2 * g.strideA2;
+    g.B += b1 * g.strideB + b2 * g.strideB2;
+    g.C += b1 * g.strideC + b2 * g.strideC2;
+  }
+  // tile of this workgroup: as gemm_dma_kernel
+  const int64_t mt = (g.M + TM - 1) / TM, ntl = (g.N + TN - 1) / TN, ntot = mt * ntl;
+  int64_t tm_i, tn_i;
+  {
+    const int64_t b = blockIdx.x;
+    if (g.b_lower) {
+      tn_i = b / mt; tm_i = b % mt;
+    } else if (g.a_lower) {
+      tm_i = mt - 1 - b / ntl; tn_i = b % ntl;
+    } else {
+      const int64_t t = ntot % 8 == 0 && !g.lower_only ? (b % 8) * (ntot / 8) + b / 8 : b;
+      tm_i = t / ntl; tn_i = t % ntl;
+    }
+  }
+  const int64_t m0 = tm_i * TM, n0 = tn_i * TN;
+  if (g.lower_only && m0 + TM - 1 < n0) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WGN, wn = wave % WGN;
+
+  const int64_t kbeg = g.b_lower ? (n0 / LKK) * LKK : 0;
+  const int64_t kend = g.a_lower ? (m0 + TM < g.K ? m0 + TM : g.K) : g.K;
+  const int64_t nst = kend > kbeg ? (kend - kbeg + LKK - 1) / LKK : 0;
+
+  // This thread's units.  [row][k] operands: row idx / 4, chunk idx % 4 (a row's
+  // 128 bytes go to four lanes); [k][n]: column idx % TN, chunk idx / TN.  A
+  // chunk is the 8 k a lane gives an MFMA, two runs of four from k_of on and 8
+  // further.  Rows past the end repeat the last one: their results are not
+  // stored.
+  auto k_of = [](int kc) __attribute__((always_inline)) { return 16 * (kc >> 1) + 4 * (kc & 1); };
+  uint32_t a_off[UA], b_off[UB];
+  int a_lds[UA], b_lds[UB], a_k[UA], b_k[UB];
+  const uint32_t b_row = (uint32_t)g.ldb * 4;
+#pragma unroll
+  for (int u = 0; u < UA; ++u) {
+    const int idx = u * NTH + tid, row = idx >> 2, kc = idx & 3;
+    const int64_t rc = m0 + row < g.M ? row : g.M - 1 - m0;
+    a_off[u] = (uint32_t)(rc * g.lda * 4) + 4 * k_of(kc);
+    a_lds[u] = kc * ASTR + row * 16;
+    a_k[u] = k_of(kc);
+  }
+#pragma unroll
+  for (int u = 0; u < UB; ++u) {
+    const int idx = u * NTH + tid;
+    const int row = BT ? idx >> 2 : idx % TN, kc = BT ? idx & 3 : idx / TN;
+    const int64_t rc = n0 + row < g.N ? row : g.N - 1 - n0;
+    b_off[u] = BT ? (uint32_t)(rc * g.ldb * 4) + 4 * k_of(kc) : (uint32_t)(rc * 4) + k_of(kc) * b_row;
+    b_lds[u] = BOFF + kc * BSTR + row * 16;
+    b_k[u] = k_of(kc);
+  }
+  const float* a_base = g.A + m0 * g.lda;
+  const float* b_base = BT ? g.B + n0 * g.ldb : g.B + n0;
+  struct Regs { f32x4_t a[UA][2], b[UB][2]; };
+  auto at = [](const float* p, uint32_t off) __attribute__((always_inline)) {
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + off);
+  };
+  // The 32 k from k0 on.  A last stage past K (a multiple of 4) reads the
+  // stage's first k in place of those past it, which the split then clears.
+  auto load = [&](Regs& r, int64_t k0) __attribute__((always_inline)) {
+    const int lim = (int)(g.K - k0 < LKK ? g.K - k0 : LKK);
+    const float* b_k0 = BT ? b_base + k0 : b_base + k0 * g.ldb;
+#pragma unroll
+    for (int u = 0; u < UA; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const bool ok = a_k[u] + 8 * h < lim;
+        r.a[u][h] = *reinterpret_cast<const f32x4_t*>(at(a_base + k0, ok ? a_off[u] + 32 * h : a_off[u] - 4 * a_k[u]));
+      }
+#pragma unroll
+    for (int u = 0; u < UB; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const bool ok = b_k[u] + 8 * h < lim;
+        if (BT) {
+          r.b[u][h] =
+              *reinterpret_cast<const f32x4_t*>(at(b_k0, ok ? b_off[u] + 32 * h : b_off[u] - 4 * b_k[u]));
+        } else {
+          const uint32_t off = ok ? b_off[u] : b_off[u] - b_k[u] * b_row;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            r.b[u][h][e] = *at(b_k0, off + (uint32_t)(8 * h + e < lim ? 8 * h + e : lim - 1) * b_row);
+        }
+      }
+  };
+  auto clear_tail = [&](Regs& r, int64_t k0) __attribute__((always_inline)) {
+    if (k0 + LKK > g.K) {
+      const int lim = (int)(g.K - k0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+          for (int u = 0; u < UA; ++u) r.a[u][h][e] = keep_if(r.a[u][h][e], a_k[u] + 8 * h < lim);
+#pragma unroll
+          for (int u = 0; u < UB; ++u) r.b[u][h][e] = keep_if(r.b[u][h][e], b_k[u] + 8 * h < lim);
+        }
+    }
+  };
+  auto split_only = [&](Regs& r, char* sl) __attribute__((always_inline)) {
+    bf16x8_t o[3];
+#pragma unroll
+    for (int u = 0; u < UA; ++u) {
+      split_x6(r.a[u][0], r.a[u][1], o);
+#pragma unroll
+      for (int t = 0; t < 3; ++t) *reinterpret_cast<bf16x8_t*>(sl + t * APL + a_lds[u]) = o[t];
+    }
+#pragma unroll
+    for (int u = 0; u < UB; ++u) {
+      split_x6(r.b[u][0], r.b[u][1], o);
+#pragma unroll
+      for (int t = 0; t < 3; ++t) *reinterpret_cast<bf16x8_t*>(sl + t * BPL + b_lds[u]) = o[t];
+    }
+  };
+
+  auto split_store = [&](Regs& r, int64_t k0, char* sl) __attribute__((always_inline)) {
+    clear_tail(r, k0);
+    split_only(r, sl);
+  };
+
+  f32x16_t acc[MB * NB2];
+#pragma unroll
+  for (int a = 0; a < MB * NB2; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[a][r] = 0.f;
+  const int half = lane >> 5, l32 = lane & 31;
+  const int a_rd = half * ASTR + (wm * WTM + l32) * 16, b_rd = BOFF + half * BSTR + (wn * WTN + l32) * 16;
+  // the six products of a stage's two 16-deep slices, term-major so that
+  // consecutive MFMAs update different accumulators
+  auto multiply = [&](const char* sl) __attribute__((always_inline)) {
+    constexpr int TA[6] = {1, 2, 0, 1, 0, 0}, TB[6] = {1, 0, 2, 0, 1, 0};
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      bf16x8_t fa[MB][3], fb[NB2][3];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+#pragma unroll
+        for (int bm = 0; bm < MB; ++bm)
+          fa[bm][t] = *reinterpret_cast<const bf16x8_t*>(sl + t * APL + 2 * s * ASTR + a_rd + bm * 512);
+#pragma unroll
+        for (int bn = 0; bn < NB2; ++bn)
+          fb[bn][t] = *reinterpret_cast<const bf16x8_t*>(sl + t * BPL + 2 * s * BSTR + b_rd + bn * 512);
+      }
+#pragma unroll
+      for (int t = 0; t < 6; ++t)
+#pragma unroll
+        for (int bm = 0; bm < MB; ++bm)
+#pragma unroll
+          for (int bn = 0; bn < NB2; ++bn)
+            acc[bm * NB2 + bn] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[bm][TA[t]], fb[bn][TB[t]], acc[bm * NB2 + bn], 0, 0, 0);
+    }
+  };
+  // LDS reads and writes done, every wave here (the loads into registers may
+  // be in flight)
+  auto sync = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  if (nst > 0) {
+    Regs r0;
+    load(r0, kbeg);
+    if constexpr (HALVES) {
+      split_store(r0, kbeg, lds);
+      if (nst > 1) load(r0, kbeg + LKK);
+      sync();
+      // each half of the waves alternates between the two, the second half
+      // beginning with the split; both meet once a stage
+      const bool split_first = wave >= 4;
+      bool skip = split_first;
+      for (int64_t m = 0, n = 0;;) {
+        if (!skip) {
+          multiply(lds + (m & 1) * STAGE);
+          ++m;
+          if (split_first) {
+            sync();
+            if (m == nst) break;
+          }
+        }
+        skip = false;
+        if (n + 1 < nst) {
+          split_store(r0, kbeg + (n + 1) * LKK, lds + ((n + 1) & 1) * STAGE);
+          if (n + 2 < nst) load(r0, kbeg + (n + 2) * LKK);
+        }
+        ++n;
+        if (!split_first) {
+          sync();
+          if (n == nst) break;
+        }
+      }
+    } else if constexpr (DEEP) {
+      // a workgroup or two on a CU: the loads two stages ahead, in two sets of
+      // registers, and one barrier a stage.  Past the last stage that one is
+      // loaded and split again, unread: without branches around them the older
+      // set's loads can be waited for while the newer's stay in flight.
+      Regs r1;
+      auto k_at = [&](int64_t st) __attribute__((always_inline)) { return kbeg + (st < nst ? st : nst - 1) * LKK; };
+      load(r1, k_at(1));
+      split_store(r0, kbeg, lds);
+      load(r0, k_at(2));
+      sync();
+      auto stage = [&](Regs& r, int64_t st, int buf) __attribute__((always_inline)) {
+        clear_tail(r, k_at(st + 1));
+        multiply(lds + buf * STAGE);
+        split_only(r, lds + (buf ^ 1) * STAGE);
+        load(r, k_at(st + 3));
+        // all LDS reads, then an MFMA (32 cycles) and the VALU instructions that
+        // go beside it, in turn
+        __builtin_amdgcn_sched_group_barrier(0x100, 6 * (MB + NB2), 0);
+#pragma unroll
+        for (int i = 0; i < 12 * MB * NB2; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, (44 * (UA + UB) + 30) / (12 * MB * NB2), 0);
+        }
+        sync();
+      };
+      for (int64_t st = 0; st < nst; st += 2) {
+        stage(r1, st, 0);
+        if (st + 1 < nst) stage(r0, st + 1, 1);
+      }
+    } else {
+      for (int64_t st = 0; st < nst; ++st) {
+        split_store(r0, kbeg + st * LKK, lds);
+        if (st + 1 < nst) load(r0, kbeg + (st + 1) * LKK);
+        sync();
+        multiply(lds);
+        sync();
+      }
+    }
+  }
+
+  constexpr int NBLK = MB * NB2;
+  float cv[NBLK * 16];
+  auto gm_of = [&](int bm, int r) { return m0 + wm * WTM + bm * 32 + 8 * (r >> 2) + 4 * half + (r & 3); };
+  auto gn_of = [&](int bn) { return n0 + wn * WTN + bn * 32 + l32; };
+  if (g.beta != 0.f) {
+#pragma unroll
+    for (int bm = 0; bm < MB; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < NB2; ++bn)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int64_t gm = gm_of(bm, r), gn = gn_of(bn);
+          cv[(bm * NB2 + bn) * 16 + r] = g.C[(gm < g.M ? gm : g.M - 1) * g.ldc + (gn < g.N ? gn : g.N - 1)];
+        }
+  }
+  // (masked stores at C's edges and the diagonal only: as gemm_dma_kernel)
+  const bool whole = m0 + TM <= g.M && n0 + TN <= g.N && (!g.lower_only || m0 >= n0 + TN - 1);
+  auto put = [&](auto masked) __attribute__((always_inline)) {
+#pragma unroll
+    for (int bm = 0; bm < MB; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < NB2; ++bn)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int64_t gm = gm_of(bm, r), gn = gn_of(bn);
+          if (!decltype(masked)::value || (gm < g.M && gn < g.N && (!g.lower_only || gm >= gn))) {
+            const float prod = g.alpha * acc[bm * NB2 + bn][r];
             g.C[gm * g.ldc + gn] = g.beta == 0.f ? prod : g.beta * cv[(bm * NB2 + bn) * 16 + r] + prod;
           }
         }
@@ -2171,46 +2389,39 @@ int gemm_f32(const GemmArgs& g, bool b_trans, int batch, hipStream_t stream) {
                    (b_trans || g.N % 4 == 0) && g.strideA % 4 == 0 && g.strideB % 4 == 0 && g.strideA2 % 4 == 0 &&
                    g.strideB2 % 4 == 0;
   if ((g.K >= 256 || (g.K >= 128 && g.x6 == 2)) && v16 && batch <= 65535 &&
-      ((g.M + 63) / 64) * ((g.N + 63) / 64) < (1ll << 31) && g.x6 && x6_enabled()) {
-    // fp32-accurate bf16 products: 256 x 128 tiles on eight waves or 128 x
-    // 128 on four (64 x 64 per wave) when they fill the CUs, else 64 x 128
-#define MQ_DMA_X6(TM, TN, WM, WN, NSX)                                                                              \
+      ((g.M + 63) / 64) * ((g.N + 63) / 64) < (1ll << 31) && g.x6 && x6_enabled() &&
+      g.lda < (1 << 20) && g.ldb < (1 << 20)) {   // 32-bit offsets within a tile
+    // fp32-accurate bf16 products
+#define MQ_X6(TM, TN, WM, WN)                                                                                  \
   do {                                                                                                         \
     dim3 grid((unsigned)(((g.N + TN - 1) / TN) * ((g.M + TM - 1) / TM)), 1, (unsigned)batch);                  \
     if (b_trans)                                                                                               \
-      hipLaunchKernelGGL((gemm_dma_kernel<TM, TN, WM, WN, true, NSX, true>), grid, dim3(64 * WM * WN), 0, stream, g); \
+      hipLaunchKernelGGL((gemm_x6_kernel<TM, TN, WM, WN, true>), grid, dim3(64 * WM * WN), 0, stream, g);      \
     else                                                                                                       \
-      hipLaunchKernelGGL((gemm_dma_kernel<TM, TN, WM, WN, false, NSX, true>), grid, dim3(64 * WM * WN), 0, stream, g); \
+      hipLaunchKernelGGL((gemm_x6_kernel<TM, TN, WM, WN, false>), grid, dim3(64 * WM * WN), 0, stream, g);     \
   } while (0)
-    // (eight waves of 64 x 32, and rings of four to six stages, measured no
-    // faster: the splits' VALU work bounds the kernel, not the loads)
-    // (triangular and lower-only products: the smaller tile, whose K
-    // ranges and diagonal waste are finer)
-    // 256 x 128 tiles on eight waves (64 x 64 each, two per SIMD: one
-    // wave's splits run beside the other's MFMAs) for products that fill
-    // the CUs with them: the d = 14336 solve's lazy updates 8.53 -> 8.04 ms,
-    // its Cholesky chain 20.4 -> 19.5 ms (lower-only rank-512 updates) ->
-    // 18.4 ms (triangular doubling products), 128 batched d = 2048 chains
-    // 10.89 -> 10.66 ms, C0 unchanged
-    // The tile whose rounds on the CUs, in 64 x 128-tile units of work, are
-    // fewest wins, the eight-wave tile credited with the 8 % it measured
-    // faster per tile (C0's 4096 x 3072 update: 384 wide tiles are two
-    // rounds, 768 of 128 x 128 three, so the latter stays)
-    const bool plain = !g.lower_only && !g.a_lower && !g.b_lower;
-    const int64_t cus = gemm_cus();
-    auto rounds = [cus](int64_t tiles) { return (tiles + cus - 1) / cus; };
-    const int64_t t256 = ((g.M + 255) / 256) * ((g.N + 127) / 128) * batch;
-    const int64_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
-    const int64_t t64 = ((g.M + 63) / 64) * ((g.N + 127) / 128) * batch;
-    const bool mid = plain && t128 >= 256;   // 128 x 128 on four waves, else 64 x 128
-    const int64_t alt = mid ? 200 * rounds(t128) : 100 * rounds(t64);
-    if (t256 >= (plain ? 128 : 256) && 400 * rounds(t256) * 100 <= 108 * alt)
-      MQ_DMA_X6(256, 128, 4, 2, 3);
-    else if (mid)
-      MQ_DMA_X6(128, 128, 2, 2, 3);
+    // Which tile, by how many of them a CU gets (those of a lower-only product
+    // above the diagonal exit at once, so half count).  4096 rows, K = 1024, by
+    // N, in us (256 x 128 | 128 x 128 | 64 x 128):
+    //   N = 1024   79 |  68 |  59   one 128 x 128 tile a CU has nothing beside it
+    //   N = 2048   83 |  92 | 114   one round of wide tiles, full
+    //   N = 3072  159 | 131 | 173   two rounds of wide tiles, the second half empty
+    // and 64 products of 768 x 1536, K = 512, 446 | 402 | 565: over many rounds
+    // the clock sinks to what the chip's power allows (1.5 GHz over 0.8 ms), and
+    // the tiles two to a CU, whose rounds do not all end at once, come out
+    // ahead.  192 .. 204 TFLOP/s are 1150 .. 1230 on the bf16 MFMA, the rate of
+    // a large library product here.  Triangular operands: a wide tile's K range
+    // is the coarser one.
+    const int64_t cus = gemm_cus(), half = g.lower_only ? 2 : 1;
+    const int64_t t256 = ((g.M + 255) / 256) * ((g.N + 127) / 128) * batch / half;
+    const int64_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128) * batch / half;
+    if (!g.a_lower && !g.b_lower && t256 <= cus && 10 * t256 >= 7 * cus)
+      MQ_X6(256, 128, 4, 2);
+    else if (2 * t128 >= 3 * cus)
+      MQ_X6(128, 128, 2, 2);
     else
-      MQ_DMA_X6(64, 128, 2, 2, 3);
-#undef MQ_DMA_X6
+      MQ_X6(64, 128, 2, 2);
+#undef MQ_X6
     MQ_LAUNCH_CHECK();
     return MI355Q_OK;
   }
