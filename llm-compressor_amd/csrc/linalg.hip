@@ -1558,17 +1558,18 @@ __global__ __launch_bounds__(PNT) void potf2_inv_kernel(const float* F, int64_t 
 // ticks the waiter marks its matrix MI355Q_TIMEOUT and raises the abort word,
 // after which every wait returns at once and all workgroups drain.
 //
-// Flags (int32, per matrix in its workspace): lf[i T + j] = 2 when tile
-// (i, j) of F holds L_ij (i > j) or X_jj is in X (i == j), 1 when the
-// diagonal tile holds A_jj fully updated; xf[i T + j] = 1 when X_ij (i > j)
-// is in X; st[4 c + s] = 1 when strip s of L_{c+1,c} is out; nl[c] and
-// nd[c] count the strips of column c done with L and with the diagonal
-// update (the last one sets the tile's lf).  Matrix 0's area then holds the
+// Flags (int32, per matrix in its workspace): lf[i T + j] = 1 when tile
+// (i, j) of F holds L_ij (i > j) or X_jj is in X (i == j); xf[i T + j] = 1
+// when X_ij (i > j) is in X; st[4 c + s] = 1 when strip s of L_{c+1,c} is
+// out; nd[c] counts the strips of A_{c+1,c+1} fully updated, which the chain
+// waits for itself; nl[c] counts the strips done with both, the last of which
+// sets L_{c+1,c}'s lf (for H tasks and later S, which need it only after the
+// chain's next factorisation).  Matrix 0's area then holds the
 // task counter and the abort word.  diag_damp_kernel clears them.
 constexpr int DSM = 2 * NB * LP + 3 * SB * LT + 2 * SB;  // LDS floats (157 KB: one workgroup per CU)
 
 constexpr int DLB = NB + 32;                             // LDS row stride of [k][n] tiles
-constexpr int DAG_LF_ACC = 1, DAG_LF_FINAL = 2;
+constexpr int DAG_LF_FINAL = 1;
 // flags per matrix: lf, xf (T^2 each), st (4 T), nl, nd (T each), then counter and abort word
 __host__ __device__ constexpr int64_t dag_nflags(int64_t T) { return 2 * T * T + 6 * T + 2; }
 
@@ -1735,10 +1736,21 @@ __device__ __forceinline__ void dag_mma_tri(DagAcc& acc, const float* la, const 
   }
 }
 
+// Every wave's stores have reached the L2 (their acknowledgements count down
+// vmcnt): one release by thread 0 then writes all of them back.  (A release
+// fence in every wave before it is a second write-back in line.  The chain of
+// d = 4096 is 31 steps of four such hand-overs each, so what stands between
+// them counts: with one write-back each, the strips' flags polled side by
+// side and the diagonal tile's count read by the chain itself, the launch
+// takes 1190 us, 1360 before; 20 of the 37 us of a step are the diagonal
+// tile's factorisation.)
+__device__ __forceinline__ void dag_stores_done() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
 // Publish: every wave's stores complete and written back, then the flag.
 __device__ __forceinline__ void dag_publish(gint* flag, int v) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  __syncthreads();
+  dag_stores_done();
   if (threadIdx.x == 0) __hip_atomic_store(flag, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -1748,17 +1760,29 @@ __device__ __forceinline__ void dag_publish(gint* flag, int v) {
 __shared__ __attribute__((aligned(16))) float dag_smem[DSM];
 __shared__ int dag_word;
 
-// Wait until *flag >= v; false when the wait was abandoned (time-out or
-// abort).  Thread 0 polls; the workgroup leaves together.
-__device__ __forceinline__ bool dag_wait(const gint* flag, int v, const DagParams& p, int b) {
+// Wait until the n flags from `flag` on are all >= v; false when the wait was
+// abandoned (time-out or abort).  Thread 0 polls them side by side; the
+// workgroup leaves together.
+__device__ __forceinline__ bool dag_wait(const gint* flag, int v, const DagParams& p, int b, int n = 1) {
   if (threadIdx.x == 0) {
     gint* abort_word = (gint*)p.flags + dag_nflags(p.T) - 1;
     int ok = 1;
-    if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) {
+    auto low = [&]() __attribute__((always_inline)) {
+      int f[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        f[q] = __hip_atomic_load(flag + (q < n ? q : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return min(f[0], min(f[1], f[2]));
+    };
+    auto one = [&]() __attribute__((always_inline)) {
+      return __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto reached = [&]() __attribute__((always_inline)) { return (n > 1 ? low() : one()) >= v; };
+    if (!reached()) {
       const uint64_t t0 = wall_clock64();
       for (;;) {
         __builtin_amdgcn_s_sleep(1);
-        if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= v) break;
+        if (reached()) break;
         if (__hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
           p.status[b] = MI355Q_TIMEOUT;  // this matrix's results are incomplete too
           ok = 0;
@@ -1825,6 +1849,7 @@ __device__ __noinline__ void dag_chain(DagParams p, int b) {
   const int T = p.T;
   const int64_t d = p.d;
   gint* lf = dag_lf(p, b);
+  const gint* nd = lf + 2 * T * T + 5 * T;
   float* a = dag_smem;
   float* x = dag_smem + NB * LP;
   float* t = dag_smem + 2 * NB * LP;
@@ -1833,7 +1858,7 @@ __device__ __noinline__ void dag_chain(DagParams p, int b) {
   for (int j = 0; j < T; ++j) {
     const int r0 = threadIdx.x >> 5, c = 4 * (threadIdx.x & 31);
     // (the first diagonal tile has no update: as prepared)
-    if (j >= 1 && !dag_wait(lf + j * T + j, DAG_LF_ACC, p, b)) return;
+    if (j >= 1 && !dag_wait(nd + j - 1, 4, p, b)) return;
     dag_fetch(dag_tile(p.F, p, b, j, j), d, v);
 #pragma unroll
     for (int i = 0; i < 16; ++i)
@@ -1960,12 +1985,8 @@ __device__ __noinline__ void dag_task_s(DagParams p, int b, int c, int s) {
   }
   dag_each_strip([&](int r, int row, int col) { sub[row * d + col] = s0[r]; });
   dag_publish(st + 4 * c + s, 1);
-  if (threadIdx.x == 0 &&
-      __hip_atomic_fetch_add(nl + c, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == 3)
-    __hip_atomic_store(lf + (c + 1) * T + c, DAG_LF_FINAL, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
   // A_{c+1,c+1}[s][0..s] -= L[s] L[0..s]^T
-  for (int q = 0; q < s; ++q)
-    if (!dag_wait(st + 4 * c + q, 1, p, b)) return;
+  if (s > 0 && !dag_wait(st + 4 * c, 1, p, b, s)) return;
   // (this workgroup read its strip's rows of A_{c+1,c} before storing them
   // as L: drop any cached copy before reading them back)
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -1976,12 +1997,14 @@ __device__ __noinline__ void dag_task_s(DagParams p, int b, int c, int s) {
     dag_mma_strip<false>(d0, d1, s0, s1, pa, pbd, pbd, NB / 2, -1.f);
     dag_each_strip([&](int r, int row, int col) { dia[row * d + col] = d0[r] + d1[r]; });
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  __syncthreads();
-  if (threadIdx.x == 0 &&
-      __hip_atomic_fetch_add(nd + c, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == 3)
-    __hip_atomic_store(lf + (c + 1) * T + c + 1, DAG_LF_ACC, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-  // off the chain's path: hinv's diagonal tile for X_cc, still in lb
+  dag_stores_done();
+  if (threadIdx.x == 0) {
+    __hip_atomic_fetch_add(nd + c, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    // off the chain's path from here: L_{c+1,c} complete with its last strip
+    if (__hip_atomic_fetch_add(nl + c, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == 3)
+      __hip_atomic_store(lf + (c + 1) * T + c, DAG_LF_FINAL, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // hinv's diagonal tile for X_cc, still in lb
   if (s == 0) dag_hinv_diag(p, b, c, lb);
 }
 
