@@ -471,16 +471,20 @@ __global__ __launch_bounds__(GNT, 2) void gemm_k128_small_kernel(GemmArgs g) {
 
 // In-place K = N = 128 products C = alpha A B^T with C the rows of A (the
 // Cholesky panel solve F[r, k0:k0+128] <- F[r, k0:k0+128] linv^T).  Each
-// workgroup owns whole rows of C - a 32 x 128 tile, all of N - and has read
-// all of its A rows before any of its waves writes, so no workgroup reads
+// workgroup owns whole rows of C - 32 x 128 tiles, all of N - and has read
+// all of a tile's A rows before any of its waves writes, so no workgroup reads
 // what another one overwrites.  (Two 64-column tiles per row tile would let
 // one workgroup overwrite rows its neighbour had not read yet, which happens
 // whenever the two do not run at the same time.)  Four waves, each a 32 x 32
-// quadrant; A [row][k] and B [n][k] in LDS, 82.6 KB.
-constexpr int RT = 32;           // rows per workgroup
+// quadrant.  B goes through LDS once into registers (a lane's 64 values), and
+// the workgroup walks its matrix's row tiles, the next tile's loads in flight
+// under this one's 64 MFMAs (4096 cycles, 1.9 us): with a workgroup per tile,
+// which loaded and staged B's 64 KB each time, that took longer than the
+// products.  The 15 solves of 64 matrices of order 2048 take 458 us, 663 before.
+constexpr int RT = 32;           // rows per tile
 
 __global__ __launch_bounds__(GNT, 1) void gemm_k128_rows_kernel(GemmArgs g) {
-  __shared__ float la[RT * KLA];
+  __shared__ float la[2][RT * KLA];
   __shared__ float lb[KT * KLA];
   {
     const int64_t bz = blockIdx.z;
@@ -490,58 +494,72 @@ __global__ __launch_bounds__(GNT, 1) void gemm_k128_rows_kernel(GemmArgs g) {
     g.C += b1 * g.strideC + b2 * g.strideC2;
   }
   const int tid = threadIdx.x, lane = tid & 63, wn = tid >> 6;
-  const int64_t m0 = (int64_t)blockIdx.y * RT;
+  const int64_t ntiles = g.M / RT;
   auto at = [](const float* base, uint32_t off) {
     return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + off);
   };
   // float4 v of a [row][k] tile covers row 8 v + tid / 32, k 4 (tid % 32)
-  f32x4_t ra[RT / 8], rb[KT / 8];
-  {
-    const uint32_t off_a = (uint32_t)((tid >> 5) * g.lda + 4 * (tid & 31)) * 4u;
-    const float* pa = g.A + m0 * g.lda;
+  const int row = tid >> 5, k4 = 4 * (tid & 31);
+  const uint32_t off_a = (uint32_t)(row * g.lda + k4) * 4u;
+  f32x4_t ra[RT / 8];
+  auto load_a = [&](int64_t t) {
+    const float* p = g.A + t * RT * g.lda;
 #pragma unroll
-    for (int v = 0; v < RT / 8; ++v) ra[v] = *reinterpret_cast<const f32x4_t*>(at(pa + 8 * v * g.lda, off_a));
-    const uint32_t off_b = (uint32_t)((tid >> 5) * g.ldb + 4 * (tid & 31)) * 4u;
-#pragma unroll
-    for (int v = 0; v < KT / 8; ++v) rb[v] = *reinterpret_cast<const f32x4_t*>(at(g.B + 8 * v * g.ldb, off_b));
-  }
-  const uint32_t off_c = (uint32_t)(4 * (lane >> 5) * g.ldc + wn * 32 + (lane & 31)) * 4u;
-  float* cbase = g.C + m0 * g.ldc;
-  float cv[16];
-  if (g.beta != 0.f) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) cv[r] = *at(cbase + (8 * (r >> 2) + (r & 3)) * g.ldc, off_c);
-  }
-  {
-    const int row = tid >> 5, k4 = 4 * (tid & 31);
+    for (int v = 0; v < RT / 8; ++v) ra[v] = *reinterpret_cast<const f32x4_t*>(at(p + 8 * v * g.lda, off_a));
+  };
+  auto store_a = [&](float* l) {
 #pragma unroll
     for (int v = 0; v < RT / 8; ++v)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) la[(8 * v + row) * KLA + k4 + e] = ra[v][e];
+      for (int e = 0; e < 4; ++e) l[(8 * v + row) * KLA + k4 + e] = ra[v][e];
+  };
+  load_a(blockIdx.y);
+  {
+    f32x4_t rb[KT / 8];
+    const uint32_t off_b = (uint32_t)(row * g.ldb + k4) * 4u;
+#pragma unroll
+    for (int v = 0; v < KT / 8; ++v) rb[v] = *reinterpret_cast<const f32x4_t*>(at(g.B + 8 * v * g.ldb, off_b));
+    store_a(la[0]);
 #pragma unroll
     for (int v = 0; v < KT / 8; ++v)
 #pragma unroll
       for (int e = 0; e < 4; ++e) lb[(8 * v + row) * KLA + k4 + e] = rb[v][e];
   }
-  __syncthreads();   // every A row of this tile is read before any C row is written
-
-  f32x16_t acc0, acc1;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc0[r] = acc1[r] = 0.f;
-  const float* pa = la + (lane & 31) * KLA + (lane >> 5);
+  const int64_t step = gridDim.y;
+  int64_t t = blockIdx.y;
+  if (t + step < ntiles) load_a(t + step);
+  __syncthreads();   // every A row of a tile is read before any C row of it is written
   const float* pb = lb + (wn * 32 + (lane & 31)) * KLA + (lane >> 5);
+  float bv[KT / 2];
 #pragma unroll
-  for (int kk = 0; kk < KT / 2; kk += 2) {
-    const float a0 = pa[2 * kk], a1 = pa[2 * kk + 2];
-    const float b0 = pb[2 * kk], b1 = pb[2 * kk + 2];
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc1, 0, 0, 0);
-  }
+  for (int kk = 0; kk < KT / 2; ++kk) bv[kk] = pb[2 * kk];
+  const uint32_t off_c = (uint32_t)(4 * (lane >> 5) * g.ldc + wn * 32 + (lane & 31)) * 4u;
+  for (int buf = 0;; buf ^= 1, t += step) {
+    float* cbase = g.C + t * RT * g.ldc;
+    float cv[16];
+    if (g.beta != 0.f) {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const float prod = g.alpha * (acc0[r] + acc1[r]);
-    const float out = g.beta == 0.f ? prod : g.beta * cv[r] + prod;
-    *const_cast<float*>(at(cbase + (8 * (r >> 2) + (r & 3)) * g.ldc, off_c)) = out;
+      for (int r = 0; r < 16; ++r) cv[r] = *at(cbase + (8 * (r >> 2) + (r & 3)) * g.ldc, off_c);
+    }
+    f32x16_t acc0, acc1;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc0[r] = acc1[r] = 0.f;
+    const float* pa = la[buf] + (lane & 31) * KLA + (lane >> 5);
+#pragma unroll
+    for (int kk = 0; kk < KT / 2; kk += 2) {
+      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(pa[2 * kk], bv[kk], acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(pa[2 * kk + 2], bv[kk + 1], acc1, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float prod = g.alpha * (acc0[r] + acc1[r]);
+      const float out = g.beta == 0.f ? prod : g.beta * cv[r] + prod;
+      *const_cast<float*>(at(cbase + (8 * (r >> 2) + (r & 3)) * g.ldc, off_c)) = out;
+    }
+    if (t + step >= ntiles) break;
+    store_a(la[buf ^ 1]);
+    if (t + 2 * step < ntiles) load_a(t + 2 * step);
+    __syncthreads();
   }
 }
 
@@ -2375,8 +2393,10 @@ int gemm_f32(const GemmArgs& g, bool b_trans, int batch, hipStream_t stream) {
     if (g.K == KT && g.N == KT && g.M % RT == 0 && g.M / RT <= 65535 && g.lda % 4 == 0 && g.ldb % 4 == 0 &&
         aligned16(g.A) && aligned16(g.B) && (batch == 1 || strides16) && (g.lda * 7 + KT) < (1 << 29) &&
         (g.ldb * 7 + KT) < (1 << 29) && (g.ldc * 31 + KT) < (1 << 29)) {
-      hipLaunchKernelGGL(gemm_k128_rows_kernel, dim3(1, (unsigned)(g.M / RT), (unsigned)batch), dim3(GNT), 0,
-                         stream, g);
+      // one workgroup per CU, the matrices' row tiles shared out among them
+      const int64_t per = (gemm_cus() + batch - 1) / batch;
+      hipLaunchKernelGGL(gemm_k128_rows_kernel, dim3(1, (unsigned)(g.M / RT < per ? g.M / RT : per), (unsigned)batch),
+                         dim3(GNT), 0, stream, g);
     } else {
       hipLaunchKernelGGL((gemm_f32_kernel<true, false>), dim3(1, (unsigned)((g.M + GBM - 1) / GBM), (unsigned)batch),
                          dim3(GNT), 0, stream, g);
