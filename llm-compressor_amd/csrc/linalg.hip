@@ -1760,7 +1760,7 @@ __device__ __forceinline__ void dag_mma_tri(DagAcc& acc, const float* la, const 
 // d = 4096 is 31 steps of four such hand-overs each, so what stands between
 // them counts: with one write-back each, the strips' flags polled side by
 // side and the diagonal tile's count read by the chain itself, the launch
-// takes 1190 us, 1360 before; 20 of the 37 us of a step are the diagonal
+// takes 1190 us, 1360 before; 17 of the 37 us of a step are the diagonal
 // tile's factorisation.)
 __device__ __forceinline__ void dag_stores_done() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
