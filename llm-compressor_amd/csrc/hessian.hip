@@ -1332,12 +1332,14 @@ void launch_reduce(const float* ws, int S, const Matrix& single, int64_t d, int6
 // The three bf16 planes of np rows of fp32 x (rows n .. np - 1 and columns d
 // .. ld - 1 zeros), eight columns per thread: h = bf16(v), m = bf16(v - h), l
 // = v - h - m, each difference exact.  Sets *unsafe for a value whose products
-// could differ from fp32 arithmetic in more than rounding: not finite, or 2^54
-// and above.  Below that no plane product overflows, and neither does a sum of
-// fewer than 2^19 of them (a call's rows), so none becomes an infinity that
-// another plane's would turn into NaN (h h' = inf, h m' = -inf from about 2^70
-// on).
-constexpr uint32_t kSplitMost = (127u + 54u) << 23;   // fp32 bits of 2^54
+// could differ from fp32 arithmetic in more than rounding: not finite, 2^54 and
+// above, or below 2^-110 and not zero.  Below 2^54 no plane product overflows,
+// and neither does a sum of fewer than 2^19 of them (a call's rows), so none
+// becomes an infinity that another plane's would turn into NaN (h h' = inf, h m'
+// = -inf from about 2^70 on).  From 2^-110 on the last of the 24 bits is at least
+// 2^-133, the least that bf16 holds (the MFMA keeps subnormal operands); below,
+// l loses bits: 2e-6 of a product's value at 2^-115, 2e-3 at 2^-125.
+constexpr uint32_t kSplitMost = (127u + 54u) << 23, kSplitLeast = (127u - 110u) << 23;   // fp32 bits
 __global__ __launch_bounds__(256) void split_planes_kernel(const float* __restrict__ x, int64_t n, int64_t d,
                                                            int64_t ldx, uint16_t* __restrict__ out, int64_t np,
                                                            int64_t ld, int vec, int* unsafe) {
@@ -1363,7 +1365,8 @@ __global__ __launch_bounds__(256) void split_planes_kernel(const float* __restri
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const uint16_t h = f32_to_bf16_bits(v[k]);
-    bad |= (__float_as_uint(v[k]) & 0x7fffffffu) >= kSplitMost;
+    const uint32_t a = __float_as_uint(v[k]) & 0x7fffffffu;
+    bad |= a != 0u && a - kSplitLeast >= kSplitMost - kSplitLeast;
     const float rest = v[k] - bf16_bits_to_f32(h);
     const uint16_t m = f32_to_bf16_bits(rest);
     const uint16_t l = f32_to_bf16_bits(rest - bf16_bits_to_f32(m));

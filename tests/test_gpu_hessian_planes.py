@@ -1,5 +1,15 @@
 """The bf16 planes of an fp32 Hessian, value by value: what they do not hold
-takes the fp32 product, as the call without a workspace does."""
+takes the fp32 product, as the call without a workspace does.
+
+Columns that share one token and no other give sums of a single product v w,
+so what each of the six plane products carries can be seen.  With h = bf16(v),
+m = bf16(v - h), l = v - h - m (|m| <= 2^-8 |v|, |l| <= 2^-17 |v|) the three
+products left out, m l', l m' and l l', are together below 1.01 2^-24 |v w|, and
+five additions to the first product, which is exact, round by at most 2^-24 of
+the sum each: 6.1 2^-24 in all, and the factor of 2 is exact.  h l', l h' or m m'
+left out is an error of up to 2^-17.  Each omission breaks the bound on these
+inputs (checked below, on the CPU).
+"""
 import ctypes as C
 
 import pytest
@@ -7,6 +17,53 @@ import torch
 
 from llmcompressor_amd import _lib as L
 from llmcompressor_amd import ops
+
+
+ULP = 2.0 ** -24
+ONE_PRODUCT = 6.1 * ULP
+PAIRS = ((0, 0), (0, 1), (1, 0), (0, 2), (2, 0), (1, 1))
+
+
+def _single_products(n, d, seed, scale=None):
+    """[n, d] with one nonzero value per column, 32 or fewer columns to a
+    token, the tokens spread over all rows; full 24-bit significands."""
+    g = torch.Generator()
+    g.manual_seed(seed)
+    v = 1 + torch.rand(d, generator=g)
+    v = torch.where(torch.rand(d, generator=g) < 0.5, -v, v)
+    if scale is not None:
+        v = v * scale
+    tokens = torch.randperm(n, generator=g)[: (d + 31) // 32]
+    x = torch.zeros(n, d)
+    x[tokens[torch.arange(d) % len(tokens)], torch.arange(d)] = v
+    return x
+
+
+def _planes(v):
+    h = v.bfloat16().float()
+    m = (v - h).bfloat16().float()
+    return h.double(), m.double(), (v - h - m).bfloat16().double()
+
+
+def _error(got, x, alpha=2.0):
+    """Largest error of an upper triangle over its own value, where that is not zero."""
+    want = torch.triu(alpha * (x.double().t() @ x.double()))
+    on = want != 0
+    assert bool((got.double()[torch.triu(~on)] == 0).all())
+    return float(((got.double() - want).abs()[on] / want.abs()[on]).max())
+
+
+@pytest.mark.parametrize("left_out", PAIRS)
+def test_bound_sees_each_product(left_out):
+    x = _single_products(640, 770, 3)
+    p = _planes(x)
+    assert torch.equal(p[0] + p[1] + p[2], x.double())
+
+    def total(pairs):
+        return torch.triu(2 * sum(p[a].t() @ p[b] for a, b in pairs))
+
+    assert _error(total(PAIRS), x) <= 1.01 * ULP
+    assert _error(total([q for q in PAIRS if q != left_out]), x) > 4 * ONE_PRODUCT
 
 
 def _fp32_product(x, alpha=2.0, H=None, beta=0.0):
@@ -24,6 +81,15 @@ def _hessian(x, alpha=2.0):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,d", [(512, 512), (640, 770), (2049, 1001), (4096, 1024)])
+def test_single_products(dev, n, d):
+    x = _single_products(n, d, n + d)
+    err = _error(_hessian(x.to(dev)).cpu(), x)
+    print(f"single products {n} x {d}: {err / ULP:.2f} ulp", flush=True)
+    assert err <= ONE_PRODUCT
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("value", [1e21, -1e25, 2.3e30, 1.7e38])
 def test_products_that_overflow(dev, value):
     """Finite values whose squares overflow: an infinity, as fp32 arithmetic gives, and no NaN."""
@@ -37,3 +103,24 @@ def test_products_that_overflow(dev, value):
     assert not torch.isnan(H).any()
     assert bool((torch.diagonal(H)[9 * torch.arange(64)] == float("inf")).all())
     assert torch.equal(H, torch.triu(_fp32_product(x)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("low", [40, 80, 100, 104, 110, 115, 120, 125])
+def test_tiny_values_keep_their_bits(dev, low):
+    """Columns of about 2^-low beside columns that bring the products back to
+    about 1: the same bound, whatever the exponent.  (Products of two tiny
+    columns underflow in fp32 arithmetic too.)"""
+    n, d = 640, 770
+    tiny = torch.arange(d) % 2 == 0
+    g = torch.Generator()
+    g.manual_seed(low)
+    up = min(low, 60)
+    x = _single_products(n, d, low, torch.where(tiny, torch.tensor(2.0) ** -low, torch.tensor(2.0) ** (up - 2)))
+    got = _hessian(x.to(dev)).cpu()
+    want = torch.triu(2 * (x.double().t() @ x.double()))
+    mixed = torch.triu(tiny.unsqueeze(0) != tiny.unsqueeze(1)) & (want != 0)
+    assert int(mixed.sum()) > 1000
+    err = float(((got.double() - want).abs()[mixed] / want.abs()[mixed]).max())
+    print(f"tiny values 2^-{low}: {err / ULP:.2f} ulp", flush=True)
+    assert err <= ONE_PRODUCT
