@@ -406,12 +406,23 @@ enum StreamMode { kDense = 0, kGrouped = 1, kGroupedGather = 2, kDenseSeg = 3, k
 
 // fp32 rows as products of bf16 planes: v = h + m + l exactly (24 bits of
 // significand in 3 x 8), and v w = h h' + h m' + m h' + h l' + l h' + m m'
-// but for terms below 2^-24 |v w| each.  The six plane products of every
-// kSplitStages stages (128 tokens) follow each other in the stage sequence,
-// so that the planes' rows stay in L2 between them.
+// but for terms below 2^-24 |v w| each.  The stages go through the rows twice:
+// with h l', l h' and m m', whose sums stay below 2^-15 of the result, then with
+// h m', m h' and h h'.  Added to a long sum of h h', m m' would round away (on the
+// diagonal it is always positive, about 2^-20 of v v'), and h l' and l h' would be
+// two more roundings at that size for every 16 tokens: with the six products side
+// by side 8192 x 8192 was 1.85e-6 from 64 bits, 16384 x 2048 1.2e-6, 512 x 8192
+// 3.9e-7; so they are 9.7e-7, 3.3e-7 and 2.2e-7 (fp32 product 1.4e-6, 2.0e-6,
+// 4.0e-7).  Time: 8192 x 4096 876 -> 845 us, 32768 x 1024 317 -> 296, 2048 x 2048
+// the same, 4096 x 1000 64 -> 67, 8192 x 8192 3.28 -> 3.32 ms, 22093 x 8200 9.0 ->
+// 9.3 (six passes are two to three times closer on wide calls and 6 .. 9 % slower:
+// full-size sums change fewer bits of an accumulator, and the chip is
+// power-limited).  Within a pass the products of every kSplitStages stages (128
+// tokens) follow each other, so that the planes' rows stay in L2 between them.
 constexpr int kSplitStages = 4, kSplitPairs = 6, kSplitTokens = kSplitStages * 32;
-// (four bits per pair: the planes of the A and of the B operand)
-constexpr uint32_t kSplitA = 0x120100u, kSplitB = 0x102010u;
+// (four bits per product, in the order above: the planes of the A and of the B
+// operand)
+constexpr uint32_t kSplitA = 0x010120u, kSplitB = 0x001102u;
 
 // One work item of the streaming kernel: tile t of matrix `mat` over token
 // split s (and part `part` of `nparts` for dense tail tiles), into partial
@@ -543,11 +554,13 @@ __device__ __forceinline__ void stream_item(const SyrkParams& p, char* ring, int
   // (xs: the row's A operand, xt: its B operand, the same row but in split mode)
   auto stage_rows = [&](int64_t sc, const char*& xs, const char*& xt, int64_t& avail) __attribute__((always_inline)) {
     if constexpr (MODE == kDenseSplit) {
-      const uint32_t G = (uint32_t)(st_begin + sc), c = G / (kSplitPairs * kSplitStages);
-      const uint32_t r = G - c * (kSplitPairs * kSplitStages), q = r / kSplitStages;
+      constexpr uint32_t HALF = kSplitPairs / 2, CH = HALF * kSplitStages;   // products of a pass, stages of a chunk
+      const uint32_t all = (uint32_t)(nst_total / 2), G0 = (uint32_t)(st_begin + sc), second = G0 >= all ? 1u : 0u;
+      const uint32_t G = G0 - second * all, c = G / CH, r = G - c * CH;
+      const uint32_t q = 4 * (second * HALF + r / kSplitStages);
       const char* x0 = reinterpret_cast<const char*>(p.x) + (int64_t)(c * kSplitStages + r % kSplitStages) * sbytes;
-      xs = x0 + (int64_t)((kSplitA >> (4 * q)) & 15u) * p.plane * 2;
-      xt = x0 + (int64_t)((kSplitB >> (4 * q)) & 15u) * p.plane * 2;
+      xs = x0 + (int64_t)((kSplitA >> q) & 15u) * p.plane * 2;
+      xt = x0 + (int64_t)((kSplitB >> q) & 15u) * p.plane * 2;
       avail = SK;   // whole stages: the planes' last rows are zeros
       return;
     }
