@@ -64,7 +64,12 @@ def hessian_syrk_(H: torch.Tensor, x: torch.Tensor, alpha: float = 2.0, beta: fl
         raise ValueError(f"H must be fp32 [{d}, {d}] row-major, got {tuple(H.shape)} {H.dtype}")
     lib = L.lib()
     dt = _HESS_DT[x.dtype]
-    ws = _ws(lib.mi355q_hessian_syrk_workspace_size(n, d, dt), x.device)
+    try:
+        ws = _ws(lib.mi355q_hessian_syrk_workspace_size(n, d, dt), x.device)
+    except torch.cuda.OutOfMemoryError:
+        if dt != L.F32:
+            raise
+        ws = None   # no room for the planes (up to about 1 GiB): the fp32 product needs none
     L.check(lib.mi355q_hessian_syrk(x.data_ptr(), dt, n, d, x.stride(0), H.data_ptr(), H.stride(0), C.c_float(alpha),
                                     C.c_float(beta), L.ptr(ws), 0 if ws is None else ws.numel(), L.stream_of(x)))
     return H

@@ -142,3 +142,21 @@ def test_no_further_from_64_bits_than_the_fp32_product(dev, n, d):
     err = [float((torch.triu(H).double() - want).norm() / want.norm()) for H in (_hessian(x), _fp32_product(x))]
     print(f"{n} x {d}: planes {err[0]:.2e}, fp32 product {err[1]:.2e}", flush=True)
     assert err[0] <= err[1]
+
+
+@pytest.mark.gpu
+def test_no_memory_for_the_planes(dev):
+    """The planes' workspace not to be had: the fp32 product, which needs none."""
+    torch.cuda.empty_cache()    # no cached block that the workspace would fit
+    x = torch.randn(65536, 1024, device=dev)
+    H = torch.zeros(1024, 1024, device=dev)
+    want = _fp32_product(x)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (32 << 20)) / total, dev)
+    try:
+        ops.hessian_syrk_(H, x, alpha=2.0, beta=0.0)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert torch.equal(H, want)
