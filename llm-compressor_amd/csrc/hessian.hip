@@ -42,6 +42,7 @@
 // chunk order afterwards (deterministic).  Items are laid out chunk-major
 // and each XCD takes a contiguous eighth of them, so the tiles of one chunk
 // run on one XCD and share its rows through that XCD's L2.
+#include <algorithm>
 #include <vector>
 
 #include "common.h"
@@ -1233,7 +1234,7 @@ int device_cus() {
   return ncu;
 }
 
-int choose_splits(int64_t n, int T, int cus) {
+int choose_splits(int64_t n, int T, int cus, bool more) {
   const int64_t s = n / 2048;
   int S = s >= 8 ? 8 : s >= 4 ? 4 : s >= 2 ? 2 : 1;
   // Wide Hessians (over two rounds of tiles) take at most 4 splits, and 4
@@ -1263,7 +1264,7 @@ int choose_splits(int64_t n, int T, int cus) {
   const auto cost = [T, stages](int k) {
     return 0.7 * (double)((stages + k - 1) / k) + (k > 1 ? 8.0 + 0.1 * T * k : 0.0);
   };
-  for (int k = 2 * best; k <= 8 && T * k <= cus && 8 * k <= stages; k *= 2)
+  for (int k = 2 * best; more && k <= 8 && T * k <= cus && 8 * k <= stages; k *= 2)
     if (cost(k) < cost(best)) best = k;
   return best;
 }
@@ -1290,12 +1291,13 @@ struct DensePlan {
   int S = 1, T = 0, tail_start = 0, tail_f = 1;
   int64_t grid = 0, slots = 0;
 };
-DensePlan plan_dense(int64_t n, int64_t d) {
+// (more: split calls whose tiles leave CUs idle further, see choose_splits)
+DensePlan plan_dense(int64_t n, int64_t d, bool more = true) {
   DensePlan pl;
   const int cus = device_cus();
   const int per_xcd = cus / kXcds > 0 ? cus / kXcds : 1;
   pl.T = upper_tiles(tiles_per_edge(d));
-  pl.S = choose_splits(n, pl.T, cus);
+  pl.S = choose_splits(n, pl.T, cus, more);
   pl.tail_start = pl.T;
   const int rem = pl.T % per_xcd;
   if (pl.S == 8 && tile_edge(d) == 256 && rem > 0 && rem <= per_xcd / 2) {
@@ -1315,6 +1317,14 @@ DensePlan plan_dense(int64_t n, int64_t d) {
     pl.slots = pl.S > 1 ? (int64_t)pl.T * pl.S : 0;
   }
   return pl;
+}
+
+inline size_t plan_bytes(const DensePlan& pl, int64_t d) { return (size_t)pl.slots * tile_floats(d) * sizeof(float); }
+// The plan for a workspace of `bytes`: with too little for the further splits
+// (a caller that knows that a short call needs none) the one without them.
+inline DensePlan plan_within(int64_t n, int64_t d, size_t bytes) {
+  const DensePlan pl = plan_dense(n, d);
+  return plan_bytes(pl, d) <= bytes ? pl : plan_dense(n, d, false);
 }
 
 template <bool F16>
@@ -1408,7 +1418,7 @@ using namespace mi355q;
 
 extern "C" size_t mi355q_hessian_workspace_size(int64_t n_tokens, int64_t d) {
   if (n_tokens <= 0 || d <= 0) return 0;
-  return (size_t)plan_dense(n_tokens, d).slots * tile_floats(d) * sizeof(float);
+  return plan_bytes(plan_dense(n_tokens, d), d);
 }
 
 namespace {
@@ -1450,9 +1460,9 @@ int hessian16_impl(const void* x_dev, bool f16, int64_t n_tokens, int64_t d, int
   }
   MQ_CHECK_ARG(x_dev != nullptr && aligned16(x_dev), "hessian: x must be non-null and 16-byte aligned");
   const int nt = tiles_per_edge(d);
-  const DensePlan pl = plan_dense(n_tokens, d);
+  const DensePlan pl = plan_within(n_tokens, d, workspace_dev ? workspace_bytes : 0);
   const int T = pl.T, S = pl.S;
-  const size_t need = mi355q_hessian_workspace_size(n_tokens, d);
+  const size_t need = plan_bytes(pl, d);
   MQ_CHECK_ARG(workspace_bytes >= need && (need == 0 || workspace_dev != nullptr),
                "hessian: workspace too small (%zu < %zu)", workspace_bytes, need);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -1479,12 +1489,13 @@ inline int64_t seg_stages(int64_t rows) { return (rows + SK - 1) / SK; }
 // Workspace of a segmented call: d >= 512 runs the non-empty segments in
 // groups of kMaxSegments, one launch over each group's padded rows; d < 512
 // runs one dense call per segment.
-size_t seg_workspace(const int64_t* rows, int nseg, int64_t d) {
+size_t seg_workspace(const int64_t* rows, int nseg, int64_t d, bool more = true) {
   size_t need = 0;
-  auto upd = [&need](size_t v) { need = v > need ? v : need; };
+  if (d <= 0) return need;
+  auto upd = [&need, d, more](int64_t n) { need = std::max(need, plan_bytes(plan_dense(n, d, more), d)); };
   if (tile_edge(d) != 256) {
     for (int k = 0; k < nseg; ++k)
-      if (rows[k] > 0) upd(mi355q_hessian_workspace_size(rows[k], d));
+      if (rows[k] > 0) upd(rows[k]);
     return need;
   }
   int in_group = 0;
@@ -1493,12 +1504,12 @@ size_t seg_workspace(const int64_t* rows, int nseg, int64_t d) {
     if (rows[k] <= 0) continue;
     stages += seg_stages(rows[k]);
     if (++in_group == kMaxSegments) {
-      upd(mi355q_hessian_workspace_size(stages * SK, d));
+      upd(stages * SK);
       in_group = 0;
       stages = 0;
     }
   }
-  if (in_group) upd(mi355q_hessian_workspace_size(stages * SK, d));
+  if (in_group) upd(stages * SK);
   return need;
 }
 
@@ -1538,7 +1549,7 @@ int hessian_seg_impl(const void* const* xs, const int64_t* rows, int nseg, mi355
   MQ_CHECK_ARG(h_dev != nullptr, "hessian: null H");
   for (int k = 0; k < nseg; ++k)
     MQ_CHECK_ARG(rows[k] == 0 || aligned16(xs[k]), "hessian segments: segment %d is not 16-byte aligned", k);
-  const size_t need = seg_workspace(rows, nseg, d);
+  const size_t need = seg_workspace(rows, nseg, d, false);
   MQ_CHECK_ARG(workspace_bytes >= need && (need == 0 || workspace_dev != nullptr),
                "hessian: workspace too small (%zu < %zu)", workspace_bytes, need);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -1564,7 +1575,7 @@ int hessian_seg_impl(const void* const* xs, const int64_t* rows, int nseg, mi355
                           stream);
     } else {
       const int64_t n_eff = stages * SK;   // the padded stages' rows
-      const DensePlan pl = plan_dense(n_eff, d);
+      const DensePlan pl = plan_within(n_eff, d, workspace_dev ? workspace_bytes : 0);
       const SyrkParams p = dense_params(tb.x[0], n_eff, d, ldx, h_dev, ldh, alpha, b, pl, workspace_dev);
       if (f16)
         hipLaunchKernelGGL((syrk_stream_kernel<true, kDenseSeg, kStreamWaves>), dim3((unsigned)pl.grid), dim3(SNT),
