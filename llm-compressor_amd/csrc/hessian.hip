@@ -416,9 +416,8 @@ enum StreamMode { kDense = 0, kGrouped = 1, kGroupedGather = 2, kDenseSeg = 3, k
 // 3.9e-7; so they are 9.7e-7, 3.3e-7 and 2.2e-7 (fp32 product 1.4e-6, 2.0e-6,
 // 4.0e-7).  Time: 8192 x 4096 876 -> 845 us, 32768 x 1024 317 -> 296, 2048 x 2048
 // the same, 4096 x 1000 64 -> 67, 8192 x 8192 3.28 -> 3.32 ms, 22093 x 8200 9.0 ->
-// 9.3 (six passes are two to three times closer on wide calls and 6 .. 9 % slower:
-// full-size sums change fewer bits of an accumulator, and the chip is
-// power-limited).  Within a pass the products of every kSplitStages stages (128
+// 9.3 (a pass for each product: two to three times closer on wide calls, 6 .. 9 %
+// slower there).  Within a pass the products of every kSplitStages stages (128
 // tokens) follow each other, so that the planes' rows stay in L2 between them.
 constexpr int kSplitStages = 4, kSplitPairs = 6, kSplitTokens = kSplitStages * 32;
 // (four bits per product, in the order above: the planes of the A and of the B
