@@ -13,11 +13,13 @@
 // GEMM whose output is rounded once and then subtracted, as in the reference.
 #include "gptq_sweep.h"
 
+#include <algorithm>
 #include <mutex>
 
 #pragma clang fp contract(off)
 
 namespace mi355q {
+int64_t gemm_cus();  // compute units (the GEMM dispatch's count)
 namespace {
 
 // One row per blockIdx.y, four consecutive output columns per thread.
@@ -126,10 +128,21 @@ __global__ void store_weight_kernel(const float* w, int64_t rows, int64_t cols, 
 constexpr int PERM_NT = 512;
 constexpr int64_t PERM_LDS = 64 << 10;  // LDS bytes of the staged rows
 
-// Rows per workgroup for rows of `bytes` LDS bytes; 0: too wide to stage.
-inline int perm_rows(int64_t bytes) {
-  const int64_t n = PERM_LDS / bytes;
-  return (int)(n > 8 ? 8 : n);
+constexpr int64_t PERM_MIN = 3 << 18;  // elements from which staging is the faster way
+
+// Rows per workgroup for rows of `bytes` LDS bytes, few enough to leave no CU
+// without one (256 x 4096 bf16 loaded on 32 workgroups of eight rows took 8.1
+// us, on 256 of one 4.7); 0: gathered straight from memory, either because a
+// row is too wide to stage or because the call is small: few workgroups then
+// read, wait and gather in turn, where the direct gather is spread over the chip
+// and takes hardly more than a launch (us, direct / staged, load bf16 | store
+// bf16 with codes: 16 x 14336 4.3 / 6.7 | 4.9 / 7.7, 64 x 8192 4.3 / 5.0 | 5.3 /
+// 5.9; from there on 64 x 14336 5.5 / 6.9 | 11.0 / 7.8, 128 x 8192 5.3 / 5.4 | 15.2
+// / 5.9, 512 x 4096 6.2 / 5.2 | 20.5 / 5.7).
+inline int perm_rows(int64_t bytes, int64_t rows, int64_t cols, int64_t batch) {
+  if (rows * batch * cols < PERM_MIN) return 0;
+  const int64_t n = PERM_LDS / bytes, most = std::max<int64_t>(rows * batch / gemm_cus(), 1);
+  return (int)std::min<int64_t>(std::min<int64_t>(n, most), 8);
 }
 
 // out[r][j] = dead[j] ? 0 : w[r][perm[j]], rows nr blockIdx.x .. (matrix
@@ -305,10 +318,10 @@ extern "C" int mi355q_gptq_load_weight_batched(const void* w_dev, mi355q_dtype w
   MQ_CHECK_ARG(rows <= 65535 && batch <= 65535, "gptq_load_weight: at most 65535 rows and matrices");
   MQ_CHECK_ARG(batch == 1 || stride_w >= rows * ldw, "gptq_load_weight: matrices overlap");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // a permutation gathers from rows staged in LDS, unless a row is too wide
-  // for that (then straight from memory: 2.6 and 4.8 times the time)
+  // a permutation gathers from rows staged in LDS, unless a row is too wide for
+  // that (then straight from memory: 2.6 and 4.8 times the time) or the call small
   const int64_t row_bytes = cols * (w_dtype == MI355Q_BF16 ? 2 : 4);
-  const int nr = perm_dev ? perm_rows(row_bytes) : 0;
+  const int nr = perm_dev ? perm_rows(row_bytes, rows, cols, batch) : 0;
   const dim3 pgrid((unsigned)(nr ? (rows + nr - 1) / nr : 1), 1, (unsigned)batch);
   if (nr && w_dtype == MI355Q_BF16)
     hipLaunchKernelGGL(load_weight_perm_kernel<uint16_t>, pgrid, dim3(PERM_NT), (size_t)(nr * row_bytes), st,
@@ -450,7 +463,7 @@ extern "C" int mi355q_gptq_store_weight_batched(const float* w_work_dev, int64_t
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool bf16 = out_dtype == MI355Q_BF16;
   const int64_t row_bytes = cols * (bf16 ? 4 : 5);
-  const int nr = invperm_dev ? perm_rows(row_bytes) : 0;
+  const int nr = invperm_dev ? perm_rows(row_bytes, rows, cols, batch) : 0;
   const dim3 pgrid((unsigned)(nr ? (rows + nr - 1) / nr : 1), 1, (unsigned)batch);
   if (nr && bf16)
     hipLaunchKernelGGL(store_weight_perm_kernel<true>, pgrid, dim3(PERM_NT), (size_t)(nr * row_bytes), st, w_work_dev,

@@ -1,7 +1,8 @@
 """Permuted weight loads and stores against plain indexing.
 
-Rows up to 64 KiB of LDS words are staged and gathered from there, wider ones
-straight from memory; both are exact copies (bf16 rounding is one conversion
+Rows up to 64 KiB of LDS words are staged and gathered from there in calls of
+3 x 2^18 elements or more; wider ones and smaller calls gather straight from
+memory.  Both are exact copies (bf16 rounding is one conversion
 of values torch rounds the same way), so everything compares bit for bit.
 """
 import pytest
@@ -15,7 +16,12 @@ pytestmark = pytest.mark.gpu
 # widths off every vector size; the widest staged rows and the first past
 # them (stores: 16384 columns to bf16, 13107 to fp32; fp32 loads 16384)
 SHAPES = [(1, 1, 8), (1, 9, 130), (3, 17, 1001), (2, 5, 4096), (1, 3, 13107), (1, 3, 13108), (1, 2, 16384),
-          (1, 2, 16388)]
+          (1, 2, 16388),
+          # staged: rows that do not fill the last workgroup's share of one to
+          # eight, widths off every vector size, the widest staged rows and the
+          # first past them, and the two sides of the least size
+          (1, 787, 1001), (1, 97, 8200), (3, 2051, 130), (5, 1031, 514), (1, 61, 13107), (1, 61, 13108),
+          (1, 49, 16384), (1, 49, 16388), (1, 1031, 8192), (1, 767, 1024), (1, 768, 1024)]
 
 
 @pytest.mark.parametrize("batch,rows,cols", SHAPES)
