@@ -15,6 +15,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import statistics
 import sys
 import time
 from pathlib import Path
@@ -122,6 +123,11 @@ def main():
     ms_step = wall * 1e3 / a.steps
     hess_ms = sum(e[0].elapsed_time(e[1]) for e in evs) / a.steps
     solve_ms = sum(e[1].elapsed_time(e[2]) for e in evs) / a.steps
+    # each step by its own events: a stall in one of them moves the mean, a
+    # slower solve the median
+    by_step = {"hessian": [e[0].elapsed_time(e[1]) for e in evs], "solve": [e[1].elapsed_time(e[2]) for e in evs],
+               "step": [e[0].elapsed_time(e[2]) for e in evs]}
+    steps_ms = {k: {"median": round(statistics.median(v), 3), "max": round(max(v), 3)} for k, v in by_step.items()}
 
     # full-size sanity: codes in range, dequantised weight = bf16(code * scale)
     codes = res.codes
@@ -297,6 +303,7 @@ def main():
                    "tokens": n_tok, "group_size": GROUP, "blocksize": 128, "damp": 0.01, "actorder": None,
                    "hessian_calls": a.hessian_calls},
         "phases_ms": {"hessian": round(hess_ms, 3), "solve": round(solve_ms, 3)},
+        "steps_ms": steps_ms,
         # the same layer calibrated through the modifiers' forward hook (64
         # calls of one 2048-token sample, staged): its Hessian time plus the solve
         "hook_path_ms_per_layer": round(hs_ms + solve_ms, 3),
