@@ -160,3 +160,38 @@ def test_no_memory_for_the_planes(dev):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0, dev)
     assert torch.equal(H, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("inf_at", [None, 5, -5], ids=["finite", "inf_in_first", "inf_in_last"])
+@pytest.mark.parametrize("beta", [0.0, 0.5, 1.0])
+@pytest.mark.parametrize("n,d", [(22093, 8192), (22272, 8200)])
+def test_several_calls_of_planes(dev, n, d, beta, inf_at):
+    """Rows whose planes would pass 1 GiB go in several calls (here 21760 rows,
+    then 333, or four whole chunks of 128): beta counts once, the planes, their
+    flag and the slots are used again, and one call may take the planes while the
+    other, whose rows hold an infinity, takes the fp32 product.  The bound is the fp32 product's own error, doubled for
+    the other order of its sum; the rows of the shorter call alone are 0.03 of H."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(n)
+    x = torch.randn(n, d, generator=g, device=dev)
+    c = 77
+    if inf_at is not None:
+        x[inf_at, c] = float("inf")
+    H0 = 100 * torch.randn(d, d, generator=g, device=dev)
+    H = ops.hessian_syrk_(H0.clone(), x, alpha=2.0, beta=beta)
+    P = _fp32_product(x, 2.0, H0.clone(), beta)
+    assert torch.equal(torch.tril(H, -1), torch.tril(H0, -1))
+    if inf_at is not None:
+        # the column meets every other one once, so its entries are the same infinities
+        assert torch.equal(H[c, c:], P[c, c:]) and torch.equal(H[:c, c], P[:c, c])
+        assert bool(torch.isinf(H[c, c:]).all())
+        x[:, c] = 0
+        for h in (H, P, H0):
+            h[c, :] = 0
+            h[:, c] = 0
+    want = torch.mm(x.t().double(), x.double()).mul_(2)
+    want.add_(H0.double(), alpha=beta).triu_()
+    err = [float((torch.triu(h).double() - want).norm() / want.norm()) for h in (H, P)]
+    print(f"{n} x {d}, beta {beta}, infinity at {inf_at}: {err[0]:.2e}, fp32 product {err[1]:.2e}", flush=True)
+    assert err[0] <= 2 * err[1]
