@@ -1257,8 +1257,8 @@ int choose_splits(int64_t n, int T, int cus, bool more) {
   // 8 stages of 32 tokens a split, while the stages saved (0.7 us each)
   // outweigh the reduction (about 8 us, and 0.1 us to write and read a
   // partial tile).  Measured against splits of at least 2048 tokens: 2048 x
-  // 256 51 -> 24 us, 2048 x 512 46 -> 27, 2048 x 1024 47 -> 33, 4096 x 1024
-  // 48 -> 34, 2048 x 2048 49 -> 32, 4096 x 2048 53 -> 40.
+  // 256 51 -> 24 us, 2048 x 512 46 -> 19, 2048 x 1024 47 -> 25, 4096 x 1024
+  // 48 -> 29, 2048 x 2048 49 -> 32, 4096 x 2048 53 -> 40.
   const int64_t stages = (n + 31) / 32;
   const auto cost = [T, stages](int k) {
     return 0.7 * (double)((stages + k - 1) / k) + (k > 1 ? 8.0 + 0.1 * T * k : 0.0);
@@ -1283,15 +1283,20 @@ inline size_t tile_floats(int64_t d) { return (size_t)tile_edge(d) * tile_edge(d
 // tiles are therefore cut into f = min(4, 32 / rem) parts per split, so the
 // last round takes 1 / f of a full one (d = 4096: T = 136, rem = 8, f = 4,
 // 4.25 rounds instead of 5).  The reduction sums their f part slots per
-// split, in part order, before adding the split.  The CU count is the
+// split, in part order, before adding the split.  Under 8192 tokens a part would
+// have fewer than 8 stages of 32, and its slot costs more than the stages saved
+// (whole / cut tails: 2048 x 512 18.6 / 26.8 us, 4096 x 768 26.0 / 31.4, 6144 x
+// 1024 33.2 / 33.8; 12288 x 512 40.0 / 31.1).  The CU count is the
 // device's (queried), so the workspace size and the launch agree on it.
 constexpr int kXcds = 8;
 struct DensePlan {
   int S = 1, T = 0, tail_start = 0, tail_f = 1;
   int64_t grid = 0, slots = 0;
 };
-// (more: split calls whose tiles leave CUs idle further, see choose_splits)
-DensePlan plan_dense(int64_t n, int64_t d, bool more = true) {
+// (more: split calls whose tiles leave CUs idle further, see choose_splits;
+// tails: the tokens from which tail tiles are cut into parts)
+constexpr int64_t kTailTokens = 8192, kSplitTailTokens = 4096;
+DensePlan plan_dense(int64_t n, int64_t d, bool more = true, int64_t tails = kTailTokens) {
   DensePlan pl;
   const int cus = device_cus();
   const int per_xcd = cus / kXcds > 0 ? cus / kXcds : 1;
@@ -1299,7 +1304,7 @@ DensePlan plan_dense(int64_t n, int64_t d, bool more = true) {
   pl.S = choose_splits(n, pl.T, cus, more);
   pl.tail_start = pl.T;
   const int rem = pl.T % per_xcd;
-  if (pl.S == 8 && tile_edge(d) == 256 && rem > 0 && rem <= per_xcd / 2) {
+  if (pl.S == 8 && n >= tails && tile_edge(d) == 256 && rem > 0 && rem <= per_xcd / 2) {
     pl.tail_f = per_xcd / rem < 4 ? per_xcd / rem : 4;
     pl.tail_start = pl.T - rem;
   }
@@ -1609,7 +1614,7 @@ namespace {
 // kDenseSplit) in calls of at most `tokens` rows, whose planes take at most
 // about 1 GiB.  Taken from 512 rows and 512 columns on: there the six
 // products, the split (10 us for 1024 x 4096, at HBM speed) and the two
-// launches around them win (fp32 product against planes: 512 x 512 51 / 36
+// launches around them win (fp32 product against planes: 512 x 512 51 / 29
 // us, 512 x 4096 177 / 93, 4096 x 1000 391 / 64, 8192 x 4096 2540 / 836, i.e.
 // 164 TFLOP/s; 256 x 4096 would be a tie).
 // Workspace: a flag, the planes, the partial slots.
@@ -1618,6 +1623,12 @@ struct SplitPlan {
   size_t planes = 0, total = 0;         // byte offset of the slots; all bytes
 };
 constexpr size_t kSplitHead = 256;
+// (a stage brings in rows of two planes, also on the diagonal, and takes longer
+// than a 16-bit one: cutting tails pays from 700 rows on.  whole / cut: 512 x 512
+// 28 / 34 us, 768 x 1000 42 / 40, 1024 x 768 42 / 38, 2048 x 512 55 / 39)
+DensePlan split_dense_plan(int64_t np, int64_t d) {
+  return plan_dense(kSplitPairs * np, d, true, kSplitTailTokens);
+}
 SplitPlan split_plan(int64_t n, int64_t d) {
   SplitPlan s;
   if (n < 512 || d < 512) return s;
@@ -1629,10 +1640,10 @@ SplitPlan split_plan(int64_t n, int64_t d) {
   s.tokens = n < most ? n : most;
   s.np = pad(s.tokens);
   s.planes = kSplitHead + (size_t)3 * s.np * s.ld * 2;
-  s.total = s.planes + mi355q_hessian_workspace_size(kSplitPairs * s.np, d);
+  s.total = s.planes + plan_bytes(split_dense_plan(s.np, d), d);
   const int64_t rest = n % s.tokens;   // the last, shorter call may split its tokens another way
   if (rest) {
-    const size_t t = s.planes + mi355q_hessian_workspace_size(kSplitPairs * pad(rest), d);
+    const size_t t = s.planes + plan_bytes(split_dense_plan(pad(rest), d), d);
     if (t > s.total) s.total = t;
   }
   return s;
@@ -1652,7 +1663,7 @@ int hessian_split_impl(const float* x, int64_t n, int64_t d, int64_t ldx, float*
     hipLaunchKernelGGL(split_planes_kernel, dim3((unsigned)((np * (s.ld / 8) + 255) / 256)), dim3(256), 0, st,
                        x + r * ldx, rows, d, ldx, planes, np, s.ld, vec, unsafe);
     const int64_t ne = kSplitPairs * np;
-    const DensePlan pl = plan_dense(ne, d);
+    const DensePlan pl = split_dense_plan(np, d);
     SyrkParams p = dense_params(planes, ne, d, s.ld, h, ldh, alpha, b, pl, ws + s.planes);
     p.plane = np * s.ld;
     p.unsafe = unsafe;

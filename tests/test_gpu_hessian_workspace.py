@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from llmcompressor_amd import _lib as L
+from llmcompressor_amd import ops
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +61,22 @@ def test_short_segments_run_without_a_workspace(dev):
     L.check(lib.mi355q_hessian_syrk_segments(ptrs, rows, 3, L.BF16, d, d, H.data_ptr(), d, C.c_float(2.0),
                                              C.c_float(0.0), None, 0, L.stream_of(x)))
     _close(H, x)
+
+
+@pytest.mark.parametrize("n,d,tiles", [(1024, 512, 3 * 4), (2048, 512, 3 * 8), (4096, 768, 6 * 8), (3072, 1280, 15 * 8),
+                                       (8192, 512, 3 * 8 * 4)])
+def test_short_calls_keep_whole_tiles(dev, n, d, tiles):
+    """Partial tiles of 256 x 256: those that the choice of the splits counts, not
+    up to four times as many; tails are cut into parts from 8192 tokens on."""
+    assert L.lib().mi355q_hessian_syrk_workspace_size(n, d, L.BF16) == tiles << 18
+
+
+@pytest.mark.parametrize("n,d", [(2080, 512), (2304, 512), (2336, 768), (8191, 512), (8192, 512), (8224, 1280)])
+def test_uneven_splits_and_parts(dev, n, d):
+    """Stages that do not divide by the splits, and the two sides of the line."""
+    x = _rows(dev, n, d)
+    H0 = torch.randn(d, d, device=dev)
+    H = ops.hessian_syrk_(H0.clone(), x, alpha=2.0, beta=0.5)
+    assert torch.equal(torch.tril(H, -1), torch.tril(H0, -1))
+    want = torch.triu(2 * (x.double().t() @ x.double()) + 0.5 * H0.double())
+    assert float((torch.triu(H).double() - want).norm() / want.norm()) <= 2e-6
