@@ -8,7 +8,7 @@ import threading
 import pytest
 import torch
 
-from llmcompressor_amd import gptq, ops, workloads
+from llmcompressor_amd import _lib, gptq, ops, workloads
 from llmcompressor_amd.observers import Observer
 from llmcompressor_amd.quant_args import QuantizationArgs
 
@@ -85,3 +85,22 @@ def test_hinv_beside_a_busy_stream_is_unchanged(dev):
         torch.cuda.synchronize()
         assert ok
         assert torch.equal(got, ref), (rep, (got - ref).abs().max().item())
+
+
+def test_launches_go_to_the_current_stream(dev):
+    """The handle that every launch is given is the current stream's, in each thread."""
+    t = torch.empty(1, device=dev)
+    a, b = torch.cuda.Stream(device=dev), torch.cuda.Stream(device=dev)
+    seen = []
+
+    def other():
+        with torch.cuda.stream(b):
+            seen.append(_lib.stream_of(t))
+
+    assert _lib.stream_of(t) == torch.cuda.current_stream(dev).cuda_stream
+    with torch.cuda.stream(a):
+        th = threading.Thread(target=other)
+        th.start()
+        th.join()
+        assert _lib.stream_of(t) == a.cuda_stream
+    assert seen == [b.cuda_stream] and a.cuda_stream != b.cuda_stream
