@@ -145,6 +145,26 @@ def test_no_further_from_64_bits_than_the_fp32_product(dev, n, d):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,d", [(1024, 512), (4096, 1000)])
+def test_columns_of_every_size_on_the_planes(dev, n, d):
+    """Columns from 2^-59 to 2^48 (below 2^54 with their largest values, above
+    2^-110 with their smallest), each to its own precision: errors over the
+    product of the two columns' norms, no larger than the fp32 product's."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(n)
+    x = torch.randn(n, d, generator=g, device=dev) * torch.pow(2.0, torch.linspace(-59, 48, d, device=dev))
+    assert float(x.abs().max()) < 2.0 ** 54 and float(x[x != 0].abs().min()) >= 2.0 ** -110
+    norm = x.double().norm(dim=0)
+    want = torch.triu(x.double().t() @ x.double())
+    on = torch.triu(torch.outer(norm, norm) > 2.0 ** -80)      # above the fp32 underflow of the sums' last bits
+    err = [float(((torch.triu(H).double() / 2 - want) / torch.outer(norm, norm))[on].norm())
+           for H in (_hessian(x), _fp32_product(x))]
+    print(f"columns of every size {n} x {d}: planes {err[0]:.2e}, fp32 product {err[1]:.2e}", flush=True)
+    assert not torch.equal(torch.triu(_hessian(x)), torch.triu(_fp32_product(x)))     # the planes took it
+    assert err[0] <= err[1]
+
+
+@pytest.mark.gpu
 def test_no_memory_for_the_planes(dev):
     """The planes' workspace not to be had: the fp32 product, which needs none."""
     torch.cuda.empty_cache()    # no cached block that the workspace would fit

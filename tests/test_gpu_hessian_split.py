@@ -2,8 +2,8 @@
 
 From 512 rows and 512 columns on an fp32 Hessian is summed from six plane
 products; below, and for values that the planes do not hold (infinities, NaN,
-magnitudes that round to infinity in bf16), by the fp32 product.  The split
-is exact (24 bits of significand in three times 8) and the dropped terms are
+magnitudes of 2^54 and above, nonzero ones below 2^-110), by the fp32 product.
+The split is exact (24 bits of significand in three times 8) and the dropped terms are
 below 2^-24 of each product, so the error against float64 is that of an fp32
 sum of n products: at most n roundings of a partial sum, i.e. n 2^-24 of sum
 |x_i x_j|, which is at most the product of the two columns' norms.
@@ -70,7 +70,8 @@ def test_values_the_planes_do_not_hold(dev, value):
 
 
 def test_small_values_keep_their_columns(dev):
-    """Columns of very different sizes (1e-18 .. 1e17: the sums stay below fp32 overflow) keep their own precision."""
+    """Columns of very different sizes (1e-18 .. 1e17: the sums stay below fp32 overflow) keep their own precision
+    (values of 2^54 and above among them: the fp32 product takes the call)."""
     n, d = 1024, 512
     x = torch.randn(n, d, device=dev) * torch.logspace(-18, 17, d, device=dev)
     H = torch.zeros(d, d, device=dev)
