@@ -77,6 +77,11 @@ int mi355q_version(void);
  * called by accumulate_hessian (:63-97); the reference's 2/n scaling is
  * alpha = 2 here plus the division by num_samples in mi355q_gptq_hinv.
  * Requirements: d % 8 == 0, ldx % 8 == 0, x 16-byte aligned.
+ * Workspace: the queried size.  Calls of fewer than 16384 tokens whose tiles
+ * leave compute units idle are split into more token ranges, one for every
+ * 256 tokens or more; a workspace that does not hold those ranges' partial
+ * sums (none, under 4096 tokens) leaves the further splits out, which changes
+ * the order of the sums.
  */
 size_t mi355q_hessian_workspace_size(int64_t n_tokens, int64_t d);
 int mi355q_hessian_syrk_bf16(const void* x_dev, int64_t n_tokens, int64_t d, int64_t ldx,
@@ -99,9 +104,9 @@ int mi355q_hessian_syrk_scaled_bf16(const void* x_dev, int64_t n_tokens, int64_t
  * 16-bit MFMA kernels above (products exact in fp32), fp32 the same kernel on
  * the rows' three bf16 planes (six products, each sum accurate as in fp32)
  * from 512 rows and 512 columns on, with the queried workspace; else, without
- * a workspace, and for values the planes do not hold, an fp32 MFMA product
- * over the upper tiles.  H = beta * H + alpha * X^T X
- * on the upper triangle, as mi355q_hessian_syrk_scaled_bf16.  x is [n_tokens,
+ * a workspace, and for rows with values the planes do not hold (not finite, of
+ * 2^54 and above, nonzero below 2^-110), an fp32 MFMA product over the upper
+ * tiles.  H = beta * H + alpha * X^T X on the upper triangle, as mi355q_hessian_syrk_scaled_bf16.  x is [n_tokens,
  * d] row-major (ldx); for the 16-bit types d % 8 == 0, ldx % 8 == 0 and x
  * 16-byte aligned.  Workspace: mi355q_hessian_syrk_workspace_size. */
 size_t mi355q_hessian_syrk_workspace_size(int64_t n_tokens, int64_t d, mi355q_dtype dtype);

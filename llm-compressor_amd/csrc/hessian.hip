@@ -1615,8 +1615,8 @@ namespace {
 // about 1 GiB.  Taken from 512 rows and 512 columns on: there the six
 // products, the split (10 us for 1024 x 4096, at HBM speed) and the two
 // launches around them win (fp32 product against planes: 512 x 512 51 / 29
-// us, 512 x 4096 177 / 93, 4096 x 1000 391 / 64, 8192 x 4096 2540 / 836, i.e.
-// 164 TFLOP/s; 256 x 4096 would be a tie).
+// us, 512 x 4096 177 / 93, 4096 x 1000 391 / 64, 8192 x 4096 2540 / 850, i.e.
+// 162 TFLOP/s; 256 x 4096 would be a tie).
 // Workspace: a flag, the planes, the partial slots.
 struct SplitPlan {
   int64_t tokens = 0, np = 0, ld = 0;   // rows per call, padded rows and columns of a plane
